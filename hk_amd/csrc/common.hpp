@@ -17,6 +17,11 @@ struct hkhip_engine {
 
 namespace hkhip {
 
+// hkhip_matvec_parts_rmsnorm, with any_type also for the types hk decodes to floats (the entry point
+// refuses those).
+int matvec_parts_rmsnorm(hkhip_engine *eng, const hkhip_mat *mats, uint32_t nparts, const float *x_dev,
+                         const float *norm_dev, float eps, uint32_t n, float *const *ys, const float *const *biases,
+                         int mode, bool any_type);
 // Sets the thread's hkhip_last_error() message and returns code.
 int set_error(int code, const char *fmt, ...);
 
@@ -26,9 +31,13 @@ inline uint64_t align256(uint64_t x) { return (x + 255) & ~uint64_t(255); }
 
 // The formats whose products decode the weights to floats (fallback.hip).
 __host__ __device__ constexpr bool fallback_type(int t) {
-    return t == HKHIP_Q2_K || t == HKHIP_Q3_K || t == HKHIP_IQ2_XXS || t == HKHIP_IQ2_XS || t == HKHIP_IQ2_S ||
-           t == HKHIP_IQ3_XXS || t == HKHIP_IQ3_S || t == HKHIP_IQ1_S || t == HKHIP_IQ1_M || t == HKHIP_TQ1_0 ||
-           t == HKHIP_TQ2_0 || t == HKHIP_MXFP4 || t == HKHIP_NVFP4;
+    return t == HKHIP_IQ2_XXS || t == HKHIP_IQ2_XS || t == HKHIP_IQ2_S || t == HKHIP_IQ3_XXS || t == HKHIP_IQ3_S ||
+           t == HKHIP_IQ1_S || t == HKHIP_IQ1_M || t == HKHIP_TQ1_0 || t == HKHIP_TQ2_0 || t == HKHIP_NVFP4;
+}
+// The formats hk decodes to floats (src/format.zig:71-93): those, and three whose products run on
+// exact integer sums here.
+__host__ __device__ constexpr bool float_decode_type(int t) {
+    return fallback_type(t) || t == HKHIP_Q2_K || t == HKHIP_Q3_K || t == HKHIP_MXFP4;
 }
 
 // Block geometry in hk's file layout (src/quant/blocks.zig:13-40).
@@ -38,7 +47,7 @@ __host__ __device__ inline int block_elems(int t) {
     case HKHIP_MXFP4:
         return 32;
     case HKHIP_NVFP4: return 64;
-    case HKHIP_Q4_K: case HKHIP_Q5_K: case HKHIP_Q6_K: case HKHIP_IQ4_XS: return 256;
+    case HKHIP_Q4_K: case HKHIP_Q5_K: case HKHIP_Q6_K: case HKHIP_IQ4_XS: case HKHIP_Q2_K: case HKHIP_Q3_K: return 256;
     default: return fallback_type(t) ? 256 : 0;
     }
 }
@@ -81,7 +90,7 @@ inline int act_kind(int t) {
 // The 32-weight formats (A8 activations).
 __host__ __device__ constexpr bool legacy32(int t) {
     return t == HKHIP_Q8_0 || t == HKHIP_IQ4_NL || t == HKHIP_Q4_0 || t == HKHIP_Q4_1 || t == HKHIP_Q5_0 ||
-           t == HKHIP_Q5_1;
+           t == HKHIP_Q5_1 || t == HKHIP_MXFP4;
 }
 // The 4/5-bit 32-weight formats: zero point (gemm.zig:262-270), offset m, fifth bit.
 __host__ __device__ constexpr bool has_m(int t) { return t == HKHIP_Q4_1 || t == HKHIP_Q5_1; }
@@ -105,6 +114,10 @@ __host__ __device__ constexpr SideGeom side_geom(int t, uint32_t nbr) {
 //   Q6_K   quant plane: 208 B per block (ql qh sc) scale plane: d
 //   IQ4_XS quant plane: 128 B per block (qs)       side plane: the 8-B header (d, scales_h,
 //                                                   scales_l), block order
+//   Q3_K   quant plane: 96 B per block (hmask qs)  side plane: 16 B (scales[12], d, 0), block order
+//   Q2_K   quant plane: 64 B per block (qs)        side plane: 20 B (scales[16], d, dmin), block order
+//   MXFP4  quant plane: 16 B per block (qs)        scale plane: the block's power of two as the top
+//                                                   half of its f32 (exact: a bf16), as IQ4_NL's d
 //   Q4_0 / Q4_1 / Q5_0 / Q5_1  quant plane: 16 B per block (qs, file nibble order)
 //          side plane, one record per row of nbr = cols/32 blocks: d[nbr] f16, then m[nbr] f16
 //          (Q4_1, Q5_1), then, from the next 4-byte boundary, qh[nbr] u32 (Q5_0, Q5_1; bit j =
@@ -123,7 +136,9 @@ inline WLayout weight_layout(int t, uint32_t rows, uint32_t cols) {
     switch (t) {
     case HKHIP_Q4_K: L.qblock = 144; break;
     case HKHIP_Q8_0: L.qblock = 32; break;
-    case HKHIP_IQ4_NL: case HKHIP_Q4_0: case HKHIP_Q4_1: case HKHIP_Q5_0: case HKHIP_Q5_1: L.qblock = 16; break;
+    case HKHIP_Q3_K: L.qblock = 96; break;
+    case HKHIP_Q2_K: L.qblock = 64; break;
+    case HKHIP_MXFP4: case HKHIP_IQ4_NL: case HKHIP_Q4_0: case HKHIP_Q4_1: case HKHIP_Q5_0: case HKHIP_Q5_1: L.qblock = 16; break;
     case HKHIP_Q6_K: L.qblock = 208; break;
     case HKHIP_Q5_K: L.qblock = 176; break;
     case HKHIP_IQ4_XS: L.qblock = 128; break;
@@ -136,7 +151,7 @@ inline WLayout weight_layout(int t, uint32_t rows, uint32_t cols) {
     } else {
         L.scale_off = align256(L.quant_bytes);
         const uint64_t side = block_elems(t) == 32 ? uint64_t(rows) * side_geom(t, cols / 32).stride
-                            : nb * (t == HKHIP_IQ4_XS ? 8 : 2);
+                            : nb * (t == HKHIP_IQ4_XS ? 8 : t == HKHIP_Q3_K ? 16 : t == HKHIP_Q2_K ? 20 : 2);
         L.total = align256(L.scale_off + side); // the kernels read the scales as aligned words
     }
     return L;
@@ -221,13 +236,25 @@ constexpr uint32_t IQ4NL_T0 = iq4nl_word(0), IQ4NL_T1 = iq4nl_word(1), IQ4NL_T2 
                    IQ4NL_T3 = iq4nl_word(3);
 static_assert(IQ4NL_T0 == 0xBFAD9881u && IQ4NL_T3 == 0x71594535u, "codebook packing");
 
-// Four 4-bit indices (one per byte, each < 16) to four signed codebook bytes.
-__device__ __forceinline__ uint32_t iq4nl_lookup4(uint32_t idx) {
+// Four 4-bit indices (one per byte, each < 16) to four signed bytes of a 16-entry codebook (four
+// words of four).
+template <uint32_t T0, uint32_t T1, uint32_t T2, uint32_t T3> __device__ __forceinline__ uint32_t lookup4(uint32_t idx) {
     uint32_t sel = idx & 0x07070707u;
-    uint32_t lo = __builtin_amdgcn_perm(IQ4NL_T1, IQ4NL_T0, sel);
-    uint32_t hi = __builtin_amdgcn_perm(IQ4NL_T3, IQ4NL_T2, sel);
+    uint32_t lo = __builtin_amdgcn_perm(T1, T0, sel);
+    uint32_t hi = __builtin_amdgcn_perm(T3, T2, sel);
     uint32_t m = ((idx >> 3) & 0x01010101u) * 0xFFu; // 0xFF in bytes whose index is >= 8
     return (hi & m) | (lo & ~m);
+}
+__device__ __forceinline__ uint32_t iq4nl_lookup4(uint32_t idx) {
+    return lookup4<IQ4NL_T0, IQ4NL_T1, IQ4NL_T2, IQ4NL_T3>(idx);
+}
+// MXFP4's values (src/quant/tables.zig:16 kvalues_fp4): 0 1 2 3 4 6 8 12 and their negatives.
+__device__ __forceinline__ uint32_t fp4_lookup4(uint32_t idx) {
+    return lookup4<0x03020100u, 0x0C080604u, 0xFDFEFF00u, 0xF4F8FAFCu>(idx);
+}
+// A 32-weight block's scale from its 16 bits in the scale plane.
+template <int T> __device__ __forceinline__ float block_scale(uint32_t bits) {
+    return T == HKHIP_MXFP4 ? __builtin_bit_cast(float, bits << 16) : f16_bits_to_f32(bits);
 }
 
 // Four unsigned quants (one per byte, each < 128) minus a zero point z4 = z * 0x01010101 (z <
@@ -239,10 +266,11 @@ __device__ __forceinline__ uint32_t bits_to_b4(uint32_t b) { return ((b & 0xFu) 
 // Signed int8 weights of a 32-weight 4/5-bit block, four per word: word i of half hh (hh = 0
 // the low nibbles of the block's 16 bytes, weights 4i..4i+3; hh = 1 the high nibbles, weights
 // 16 + 4i..), from the block's quant word x (bytes 4i..4i+3) and fifth-bit word qh. Q4_1 and
-// Q5_1 stay unsigned (their offset is a separate term); IQ4_NL goes through the codebook.
+// Q5_1 stay unsigned (their offset is a separate term); IQ4_NL and MXFP4 go through their codebooks.
 template <int T> __device__ __forceinline__ uint32_t low_bit_word(uint32_t x, uint32_t qh, uint32_t hh, uint32_t i) {
     uint32_t n = (x >> (4 * hh)) & 0x0F0F0F0Fu;
     if constexpr (T == HKHIP_IQ4_NL) return iq4nl_lookup4(n);
+    if constexpr (T == HKHIP_MXFP4) return fp4_lookup4(n);
     if constexpr (has_qh(T)) n |= bits_to_b4(qh >> (16 * hh + 4 * i));
     if constexpr (zero_point(T) != 0) n = sub_zp4(n, uint32_t(zero_point(T)) * 0x01010101u);
     return n;
@@ -316,7 +344,11 @@ hipError_t launch_mmsk(int t, const uint8_t *w, uint32_t rows, uint32_t cols, co
                        float *y, const float *bias, int mode, hipStream_t s);
 hipError_t launch_mmsk_parts(int t, const MvPartDesc *parts, int nparts, uint32_t cols, const uint8_t *xq,
                              uint32_t n, int mode, hipStream_t s);
-// Prefill GEMM for Q6_K, Q8_0 and IQ4_NL (cols a multiple of 256).
+// Prefill GEMM for Q6_K, Q3_K and Q2_K (cols a multiple of 256).
+bool mmg_supports(int t, uint32_t rows, uint32_t cols, uint32_t n);
+hipError_t launch_mmg(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n, float *y,
+                      const float *bias, int mode, hipStream_t s);
+// Prefill GEMM for the 32-weight formats, Q5_K and IQ4_XS (cols a multiple of 256).
 bool mmx_supports(int t, uint32_t rows, uint32_t cols, uint32_t n);
 hipError_t launch_mmx(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n, float *y,
                       const float *bias, int mode, hipStream_t s);

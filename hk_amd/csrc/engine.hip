@@ -292,7 +292,7 @@ static int check_product(const hkhip_mat *m, const void *xq, float *y, uint32_t 
         return fail(HKHIP_E_BAD_ARGUMENT, "unknown mode %d", mode);
     if (mode == HKHIP_SILU_MUL && m->rows % 2)
         return fail(HKHIP_E_BAD_ARGUMENT, "silu(gate)*up needs interleaved gate/up rows (an even count)");
-    if ((act_kind(m->t) == HKHIP_ACT_Q8K || fallback_type(m->t)) && m->cols % QK_K)
+    if ((act_kind(m->t) == HKHIP_ACT_Q8K || float_decode_type(m->t)) && m->cols % QK_K)
         return fail(HKHIP_E_UNSUPPORTED_SHAPE, "cols %u: the products of this type take whole 256-value groups", m->cols);
     if (n && (!xq || !y)) return fail(HKHIP_E_BAD_ARGUMENT, "null buffer");
     return HKHIP_OK;
@@ -344,28 +344,7 @@ int hkhip_matvec_parts(hkhip_engine *eng, const hkhip_mat *mats, uint32_t nparts
 int hkhip_matvec_parts_rmsnorm(hkhip_engine *eng, const hkhip_mat *mats, uint32_t nparts, const float *x_dev,
                                const float *norm_dev, float eps, uint32_t n, float *const *ys,
                                const float *const *biases, int mode) {
-    int rc = enter(eng);
-    if (rc) return rc;
-    if (!mats || !ys || nparts < 1 || nparts > 4) return fail(HKHIP_E_BAD_ARGUMENT, "need 1..4 parts, got %u", nparts);
-    if (!x_dev || !norm_dev) return fail(HKHIP_E_BAD_ARGUMENT, "null input or norm weights");
-    MvPartDesc parts[4];
-    for (uint32_t i = 0; i < nparts; i++) {
-        if ((rc = check_product(&mats[i], x_dev, ys[i], n, mode))) return rc;
-        if (mode == HKHIP_SILU_MUL && biases && biases[i])
-            return fail(HKHIP_E_BAD_ARGUMENT, "silu(gate)*up takes no bias");
-        if (mats[i].t != mats[0].t || mats[i].cols != mats[0].cols)
-            return fail(HKHIP_E_BAD_ARGUMENT, "fused parts must share type and cols");
-        parts[i] = MvPartDesc{reinterpret_cast<const uint8_t *>(mats[i].mem), ys[i], biases ? biases[i] : nullptr,
-                              mats[i].rows};
-    }
-    if (n > 8) return fail(HKHIP_E_UNSUPPORTED_SHAPE, "the fused norm takes at most 8 tokens, got %u", n);
-    if (n == 0) return HKHIP_OK;
-    const hipError_t e = launch_mmvq_parts_norm(mats[0].t, parts, int(nparts), mats[0].cols, x_dev, nullptr, n, mode,
-                                                norm_dev, eps, eng->cur);
-    if (e == hipErrorNotSupported)
-        return fail(HKHIP_E_UNSUPPORTED_SHAPE, "no fused-norm kernel for %u tokens of %u cols", n, mats[0].cols);
-    HIP_TRY(e, "mmvq launch");
-    return HKHIP_OK;
+    return matvec_parts_rmsnorm(eng, mats, nparts, x_dev, norm_dev, eps, n, ys, biases, mode, false);
 }
 
 int hkhip_gemm(hkhip_engine *eng, const hkhip_mat *m, const void *xq_dev, float *y_dev, uint32_t n,
@@ -387,7 +366,7 @@ static uint32_t gemm_min_tokens(int t, uint32_t rows) {
     switch (t) {
     case HKHIP_Q6_K:
     case HKHIP_Q8_0: return 33;
-    case HKHIP_IQ4_NL: return 25;
+    case HKHIP_IQ4_NL: case HKHIP_MXFP4: return 25;
     case HKHIP_Q5_K: case HKHIP_Q4_0: case HKHIP_Q4_1: case HKHIP_Q5_0: case HKHIP_Q5_1: case HKHIP_IQ4_XS:
         // Measured at 9-64 tokens: with 14336 rows the GEMM beats two decode passes from 9
         // tokens; with 4096 rows (K 14336) it costs 50-120 us at any count (Q4_1 50, IQ4_XS 66,
@@ -514,3 +493,32 @@ int hkhip_gemv_iq4_nl(const void *w, const float *x, const float *bias, float *y
 }
 
 } // extern "C"
+
+int hkhip::matvec_parts_rmsnorm(hkhip_engine *eng, const hkhip_mat *mats, uint32_t nparts, const float *x_dev,
+                                const float *norm_dev, float eps, uint32_t n, float *const *ys,
+                                const float *const *biases, int mode, bool any_type) {
+    int rc = enter(eng);
+    if (rc) return rc;
+    if (!mats || !ys || nparts < 1 || nparts > 4) return fail(HKHIP_E_BAD_ARGUMENT, "need 1..4 parts, got %u", nparts);
+    if (!x_dev || !norm_dev) return fail(HKHIP_E_BAD_ARGUMENT, "null input or norm weights");
+    MvPartDesc parts[4];
+    for (uint32_t i = 0; i < nparts; i++) {
+        if ((rc = check_product(&mats[i], x_dev, ys[i], n, mode))) return rc;
+        if (mode == HKHIP_SILU_MUL && biases && biases[i])
+            return fail(HKHIP_E_BAD_ARGUMENT, "silu(gate)*up takes no bias");
+        if (mats[i].t != mats[0].t || mats[i].cols != mats[0].cols)
+            return fail(HKHIP_E_BAD_ARGUMENT, "fused parts must share type and cols");
+        parts[i] = MvPartDesc{reinterpret_cast<const uint8_t *>(mats[i].mem), ys[i], biases ? biases[i] : nullptr,
+                              mats[i].rows};
+    }
+    if (n > 8) return fail(HKHIP_E_UNSUPPORTED_SHAPE, "the fused norm takes at most 8 tokens, got %u", n);
+    if (n == 0) return HKHIP_OK;
+    if (!any_type && float_decode_type(mats[0].t))
+        return fail(HKHIP_E_UNSUPPORTED_SHAPE, "no fused-norm kernel for type 0x%02x", mats[0].t);
+    const hipError_t e = launch_mmvq_parts_norm(mats[0].t, parts, int(nparts), mats[0].cols, x_dev, nullptr, n, mode,
+                                                norm_dev, eps, eng->cur);
+    if (e == hipErrorNotSupported)
+        return fail(HKHIP_E_UNSUPPORTED_SHAPE, "no fused-norm kernel for %u tokens of %u cols", n, mats[0].cols);
+    HIP_TRY(e, "mmvq launch");
+    return HKHIP_OK;
+}

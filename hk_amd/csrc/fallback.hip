@@ -1,19 +1,16 @@
-// The formats hk decodes to floats before its dot products ("exact fallback"): Q2_K, Q3_K,
-// IQ2_XXS, IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S, IQ1_S, IQ1_M, TQ1_0, TQ2_0, MXFP4, NVFP4.
+// The formats whose products decode the weights to floats (of those that hk decodes so, its "exact
+// fallback"): IQ2_XXS, IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S, IQ1_S, IQ1_M, TQ1_0, TQ2_0, NVFP4.
 //
-// Decoders restate src/quant/dequant.zig (q2_k 80-112, q3kScales 114-128, q3_k 130-165,
-// iq2_xxs 278-294, iq2_xs 296-312, iq2_s 314-330, iq3_xxs 332-351, iq3_s 353-375, iq1_s 377-392,
-// iq1_m 394-428, ternary / tq1_0 460-488, tq2_0 490-504, e8m0Half / mxfp4 506-519, ue4m3Half /
-// nvfp4 521-548) one element at a time with the reference's float operations in its order (the
+// Decoders restate src/quant/dequant.zig (iq2_xxs 278-294, iq2_xs 296-312, iq2_s 314-330, iq3_xxs 332-351, iq3_s 353-375, iq1_s 377-392,
+// iq1_m 394-428, ternary / tq1_0 460-488, tq2_0 490-504, ue4m3Half / nvfp4 521-548) one element at a time with the reference's float operations in its order (the
 // library is built with -ffp-contract=off), so they are bit-exact. The device layout is the file
-// layout. Products follow hk's fallback dots (vecdot.zig dotCanonK 686-705, dotCanonLegacy 707-720,
-// dotGeneric 620-631): the weights against the dequantized Q8K / A8 activations (d * q), or the f32
-// input for NVFP4, summed in f32 -- the integer dot of the reference up to rounding.
+// layout. Products follow hk's fallback dots (vecdot.zig dotCanonK 686-705, dotGeneric
+// 620-631): the weights against the dequantized Q8K activations (d * q), or the f32 input for NVFP4, summed in f32 -- the integer dot of the reference up to rounding.
 //
 // Products: a wave owns up to FB_RPW output rows (pairs of rows for silu(gate)*up); for every
 // 256 inputs it first forms its lanes' four activation values per token (reading a prepared
 // buffer, or quantizing the f32 input itself with the qact arithmetic: a Q8K block is the whole
-// wave, an A8 block eight lanes), then decodes four weights of each of its rows per lane.
+// wave), then decodes four weights of each of its rows per lane.
 #include "quant.hpp"
 #include "iq_tables.inc" // the IQ codebooks (hk_amd/csrc/tables/*.bin) as __constant__ arrays
 
@@ -37,30 +34,6 @@ constexpr float IQ1S_DELTA = 0.125f; // tables.zig:18
 // Element e of one block.
 __device__ float fb_elem(int t, const uint8_t *b, uint32_t e) {
     switch (t) {
-    case HKHIP_Q2_K: { // {scales[16], qs[64], d, dmin}
-        const uint32_t n = e / 128, it = (e % 128) / 32, half = (e % 32) / 16, l = e % 16;
-        const uint32_t sc = b[8 * n + 2 * it + half];
-        const float d = ldh(b + 80), mn = ldh(b + 82);
-        const float dl = d * float(sc & 0x0F), ml = mn * float(sc >> 4);
-        return dl * float((b[16 + 32 * n + 16 * half + l] >> (2 * it)) & 3) - ml;
-    }
-    case HKHIP_Q3_K: { // {hmask[32], qs[64], scales[12], d}
-        const uint32_t n = e / 128, it = (e % 128) / 32, half = (e % 32) / 16, l = e % 16;
-        const uint32_t is = 8 * n + 2 * it + half; // scale index 0..15 (q3kScales)
-        const uint32_t a0 = ld32(b + 96), a1 = ld32(b + 100), tmp = ld32(b + 104);
-        uint32_t word;
-        switch (is / 4) {
-        case 0: word = (a0 & 0x0f0f0f0fu) | (((tmp >> 0) & 0x03030303u) << 4); break;
-        case 1: word = (a1 & 0x0f0f0f0fu) | (((tmp >> 2) & 0x03030303u) << 4); break;
-        case 2: word = ((a0 >> 4) & 0x0f0f0f0fu) | (((tmp >> 4) & 0x03030303u) << 4); break;
-        default: word = ((a1 >> 4) & 0x0f0f0f0fu) | (((tmp >> 6) & 0x03030303u) << 4); break;
-        }
-        const int sc = int(int8_t(uint8_t(word >> (8 * (is % 4)))));
-        const float dl = ldh(b + 108) * float(sc - 32);
-        const int lo = (b[32 + 32 * n + 16 * half + l] >> (2 * it)) & 3;
-        const int hi = (b[16 * half + l] & (1u << (4 * n + it))) ? 0 : 4;
-        return dl * float(lo - hi);
-    }
     case HKHIP_IQ2_XXS: { // {d, qs[64]}
         const uint32_t ib = e / 32, l = (e % 32) / 8, j = e % 8;
         const uint32_t aux1 = ld32(b + 2 + 8 * ib + 4);
@@ -140,12 +113,6 @@ __device__ float fb_elem(int t, const uint8_t *b, uint32_t e) {
         const uint32_t j = (e / 128) * 32, l = (e % 128) / 32, k = e % 32;
         return float(int((b[j + k] >> (2 * l)) & 3) - 1) * ldh(b + 64);
     }
-    case HKHIP_MXFP4: { // {e, qs[16]}
-        const uint32_t x = b[0];
-        const float d = __uint_as_float(x < 2 ? (0x00200000u << x) : (x - 1) << 23);
-        const uint32_t q = b[1 + (e % 16)];
-        return fp4v(e < 16 ? q & 0x0F : q >> 4) * d;
-    }
     case HKHIP_NVFP4: { // {d[4], qs[32]}: four 16-value sub-blocks with an unsigned E4M3 scale
         const uint32_t s = e / 16, j = e % 16;
         const uint32_t x = b[s];
@@ -187,7 +154,7 @@ struct FbArgs {
     uint32_t nparts, units, K, ntok;
     int t, mode;
     const float *x;   // f32 input [ntok][K], or null
-    const int8_t *qs; // prepared activations (A8 or Q8K planes)
+    const int8_t *qs; // prepared activations (Q8K planes)
     const float *d;
 };
 
@@ -206,7 +173,7 @@ __device__ __forceinline__ void fb_acts(const FbArgs &a, uint32_t t, uint32_t g,
         out[0] = v.x, out[1] = v.y, out[2] = v.z, out[3] = v.w;
     } else if (a.x == nullptr) {
         const uint32_t q = *reinterpret_cast<const uint32_t *>(a.qs + uint64_t(t) * K + e0);
-        const float d = a.d[(uint64_t(t) * K + e0) / (KIND == HKHIP_ACT_Q8K ? 256 : 32)];
+        const float d = a.d[(uint64_t(t) * K + e0) / 256];
 #pragma unroll
         for (int i = 0; i < 4; i++) out[i] = d * float(int8_t(uint8_t(q >> (8 * i))));
     } else {
@@ -215,7 +182,7 @@ __device__ __forceinline__ void fb_acts(const FbArgs &a, uint32_t t, uint32_t g,
         float m = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; i++) m = fmaxf(m, fabsf(v[i]));
-        if constexpr (KIND == HKHIP_ACT_Q8K) {
+        {
             // quantizeQ8K (vecdot.zig:150-180): the signed value of the first element with the
             // largest magnitude sets the scale; q = min(127, round(iscale * x)); d = 1 / iscale.
             const float amax = wave_max(m);
@@ -235,14 +202,6 @@ __device__ __forceinline__ void fb_acts(const FbArgs &a, uint32_t t, uint32_t g,
                 const int q = int(roundf(iscale * v[i]));
                 out[i] = d * float(q < 127 ? q : 127);
             }
-        } else {
-            // quantizeA8 (vecdot.zig:134-148): per 32 inputs (eight lanes) d = amax / 127.
-            float am = m;
-            for (int o = 1; o <= 4; o <<= 1) am = fmaxf(am, __shfl_xor(am, o));
-            const float d = __fdiv_rn(am, 127.0f);
-            const float id = d != 0.0f ? __fdiv_rn(1.0f, d) : 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; i++) out[i] = d * float(int(roundf(v[i] * id)));
         }
     }
 }
@@ -387,14 +346,11 @@ hipError_t launch_fb_mv(int t, const MvPartDesc *parts, int nparts, uint32_t K, 
         if (x) {
             c.x = x + uint64_t(t0) * K;
         } else {
-            const bool kq = kind == HKHIP_ACT_Q8K;
-            c.qs = reinterpret_cast<const int8_t *>(xq + (kq ? A.k_qs : A.a8_qs)) + uint64_t(t0) * K;
-            c.d = reinterpret_cast<const float *>(xq + (kq ? A.k_d : A.a8_d)) + uint64_t(t0) * K / (kq ? 256 : 32);
+            c.qs = reinterpret_cast<const int8_t *>(xq + A.k_qs) + uint64_t(t0) * K;
+            c.d = reinterpret_cast<const float *>(xq + A.k_d) + uint64_t(t0) * K / 256;
         }
         const uint32_t nt = nc == 1 ? 1 : nc == 2 ? 2 : nc <= 4 ? 4 : 8;
-        hipError_t e = kind == HKHIP_ACT_F32 ? fb_mv_launch<HKHIP_ACT_F32>(c, nt, s)
-                     : kind == HKHIP_ACT_Q8K ? fb_mv_launch<HKHIP_ACT_Q8K>(c, nt, s)
-                                             : fb_mv_launch<HKHIP_ACT_A8>(c, nt, s);
+        hipError_t e = kind == HKHIP_ACT_F32 ? fb_mv_launch<HKHIP_ACT_F32>(c, nt, s) : fb_mv_launch<HKHIP_ACT_Q8K>(c, nt, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -19,6 +19,9 @@ static mv_kernel_t kernel_for(int t, int nt) {
     case HKHIP_Q4_1: return pick<HKHIP_Q4_1>(nt);
     case HKHIP_Q5_0: return pick<HKHIP_Q5_0>(nt);
     case HKHIP_Q5_1: return pick<HKHIP_Q5_1>(nt);
+    case HKHIP_Q3_K: return pick<HKHIP_Q3_K>(nt);
+    case HKHIP_Q2_K: return pick<HKHIP_Q2_K>(nt);
+    case HKHIP_MXFP4: return pick<HKHIP_MXFP4>(nt);
     default: return nullptr;
     }
 }
@@ -35,6 +38,9 @@ static mv_kernel_t kernelr_for(int t, int nt, int c, int ks, bool norm) {
     case HKHIP_Q4_1: return mvr_pick<HKHIP_Q4_1>(nt, c, ks, norm);
     case HKHIP_Q5_0: return mvr_pick<HKHIP_Q5_0>(nt, c, ks, norm);
     case HKHIP_Q5_1: return mvr_pick<HKHIP_Q5_1>(nt, c, ks, norm);
+    case HKHIP_Q3_K: return mvr_pick<HKHIP_Q3_K>(nt, c, ks, norm);
+    case HKHIP_Q2_K: return mvr_pick<HKHIP_Q2_K>(nt, c, ks, norm);
+    case HKHIP_MXFP4: return mvr_pick<HKHIP_MXFP4>(nt, c, ks, norm);
     default: return nullptr;
     }
 }
@@ -51,6 +57,9 @@ static mv_kernel_t kernels_for(int t, int lg, int nw) {
     case HKHIP_Q4_1: return mvs_pick<HKHIP_Q4_1>(lg, nw);
     case HKHIP_Q5_0: return mvs_pick<HKHIP_Q5_0>(lg, nw);
     case HKHIP_Q5_1: return mvs_pick<HKHIP_Q5_1>(lg, nw);
+    case HKHIP_Q3_K: return mvs_pick<HKHIP_Q3_K>(lg, nw);
+    case HKHIP_Q2_K: return mvs_pick<HKHIP_Q2_K>(lg, nw);
+    case HKHIP_MXFP4: return mvs_pick<HKHIP_MXFP4>(lg, nw);
     default: return nullptr;
     }
 }
@@ -312,6 +321,12 @@ hipError_t launch_mmvq_parts_norm(int t, const MvPartDesc *parts, int nparts, ui
         for (int i = 0; i < nparts; i++) sk = sk && mmsk_supports(t, parts[i].rows, K, n);
         if (sk) return launch_mmsk_parts(t, parts, nparts, K, xq, n, mode, s);
     }
+    // Q3_K and Q2_K from 4 tokens with a prepared input: the prefill GEMM, whose smallest tiles cost the
+    // same from 1 token to 32 (14336 x 4096 at 4 / 8 tokens: Q3_K 11.8 / 11.7 us against 17.0 / 27.0 on
+    // the decode kernel; 4096 x 14336 18.6 / 18.7 against 18.7 / 30.8).
+    if (!x && n >= SK_MIN_TOKENS && nparts == 1 && (t == HKHIP_Q3_K || t == HKHIP_Q2_K) &&
+        mmg_supports(t, parts[0].rows, K, n))
+        return launch_mmg(t, parts[0].w, parts[0].rows, K, xq, n, parts[0].y, parts[0].bias, mode, s);
     MvAct act{};
     if (x) {
         act.x = x;

@@ -382,8 +382,94 @@ template <> struct MvFmt<HKHIP_Q6_K> {
     }
 };
 
-// The 32-weight formats, one block per unit, against A8: Q8_0 and IQ4_NL (vecdot.zig:235-250,
-// 369-384) signed; Q4_0 / Q5_0 with their zero point subtracted per weight (so the block sum is
+// Q3_K and Q2_K (dotCanonK, vecdot.zig:686-705, on the canonical unpack of unpack.zig:29-160): a
+// unit is 16 bytes of qs, whose four 2-bit fields hold 64 weights in Q6_K's order (field p of byte
+// 16lc + i of half n: weight 128n + 32p + 16lc + i, scale 8n + 2p + lc), so the activation side is
+// Q6_K's. The sums are exact integers: Q3_K's q - 4 goes through bsums, Q2_K's mins too.
+template <int T> struct MvK23 : MvFmt<HKHIP_Q6_K> {
+    static constexpr bool q3 = T == HKHIP_Q3_K;
+    struct W {
+        uint4 q, hm, side; // Q3_K: hmask bytes 16lc.., scales[12] and d
+        uint32_t s0, s1, dm; // Q2_K: scale bytes 8n.., d and dmin
+    };
+    __device__ static RowRef row(const uint8_t *w, const uint16_t *ws, uint32_t r, uint32_t K) {
+        return RowRef{w + uint64_t(r) * (K / 256) * (q3 ? 96 : 64), ws + uint64_t(r) * (K / 256) * (q3 ? 8 : 10)};
+    }
+    __device__ static W load(const RowRef &R, uint32_t u) {
+        const uint32_t n = (u >> 1) & 1, lc = u & 1;
+        W w;
+        if constexpr (q3) {
+            const uint8_t *blk = R.w + (u >> 2) * 96;
+            w.q = ldw(blk + 32 + 32 * n + 16 * lc);
+            w.hm = ldw(blk + 16 * lc);
+            w.side = ldw(R.ws + (u >> 2) * 8);
+        } else {
+            w.q = ldw(R.w + (u >> 2) * 64 + 32 * n + 16 * lc);
+            const uint32_t *sd = reinterpret_cast<const uint32_t *>(R.ws + (u >> 2) * 10);
+            w.s0 = sd[2 * n];
+            w.s1 = sd[2 * n + 1];
+            w.dm = sd[4];
+        }
+        return w;
+    }
+    struct P {
+        uint32_t q[16];
+        int sc[4], mn[4];
+        float d, dmin;
+    };
+    __device__ static P prep(const W &w, uint32_t u) {
+        const uint32_t n = (u >> 1) & 1, lc = u & 1;
+        P p;
+        const uint32_t qw[4] = {w.q.x, w.q.y, w.q.z, w.q.w};
+        const uint32_t hw[4] = {w.hm.x, w.hm.y, w.hm.z, w.hm.w};
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                p.q[4 * g + i] = (qw[i] >> (2 * g)) & 0x03030303u;
+                if constexpr (q3) p.q[4 * g + i] |= ((hw[i] >> (4 * n + g)) & 0x01010101u) << 2;
+            }
+            if constexpr (q3) { // scale 8n + 2g + lc (q3kScales, dequant.zig:114-128)
+                const uint32_t sh = 16 * (g & 1) + 8 * lc;
+                const uint32_t lo = ((g < 2 ? w.side.x : w.side.y) >> (sh + 4 * n)) & 0x0F;
+                const uint32_t hi = (w.side.z >> (sh + 4 * n + 2 * (g / 2))) & 3;
+                p.sc[g] = int(lo | (hi << 4)) - 32;
+            } else {
+                const uint32_t b = ((g < 2 ? w.s0 : w.s1) >> (16 * (g & 1) + 8 * lc)) & 0xFF;
+                p.sc[g] = int(b & 0x0F);
+                p.mn[g] = int(b >> 4);
+            }
+        }
+        p.d = f16_bits_to_f32((q3 ? w.side.w : w.dm) & 0xFFFF);
+        p.dmin = q3 ? 0.0f : f16_bits_to_f32(w.dm >> 16);
+        return p;
+    }
+    __device__ static void dotp(const P &p, const AU &a, float &acc, float &corr) {
+        int isum = 0, bias = 0;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            int sg = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) sg = sdot4(p.q[4 * g + i], a.q[4 * g + i], sg);
+            isum += sg * p.sc[g];
+            bias += (q3 ? p.sc[g] : p.mn[g]) * a.bs[g];
+        }
+        if constexpr (q3) {
+            acc = fmaf((float)(isum - 4 * bias), p.d * a.d, acc);
+        } else {
+            acc = fmaf((float)isum, p.d * a.d, acc);
+            corr = fmaf((float)bias, p.dmin * a.d, corr);
+        }
+    }
+    __device__ static void dot(const W &w, uint32_t u, const AU &a, float &acc, float &corr) {
+        dotp(prep(w, u), a, acc, corr);
+    }
+};
+template <> struct MvFmt<HKHIP_Q3_K> : MvK23<HKHIP_Q3_K> {};
+template <> struct MvFmt<HKHIP_Q2_K> : MvK23<HKHIP_Q2_K> {};
+
+// The 32-weight formats, one block per unit, against A8: Q8_0, IQ4_NL and MXFP4 (vecdot.zig:235-250,
+// 369-384, dotCanonLegacy 707-720) signed; Q4_0 / Q5_0 with their zero point subtracted per weight (so the block sum is
 // dotQ4_0's dpu - 8*s, dotQ5_0's - 16*s); Q4_1 / Q5_1 unsigned plus m * (d_a * s), with s the
 // block's activation sum (dotQ4_1 / dotQ5_1, 311-367).
 template <int T> struct MvLegacy {
@@ -446,7 +532,7 @@ template <int T> struct MvLegacy {
                 p.q[4 + i] = low_bit_word<T>(n4[i], qh, 1, i);
             }
         }
-        p.d = f16_bits_to_f32(w.d);
+        p.d = block_scale<T>(w.d);
         p.m = has_m(T) ? f16_bits_to_f32(w.m) : 0.0f;
         return p;
     }
@@ -468,6 +554,7 @@ template <int T> struct MvLegacy {
 };
 template <> struct MvFmt<HKHIP_Q8_0> : MvLegacy<HKHIP_Q8_0> {};
 template <> struct MvFmt<HKHIP_IQ4_NL> : MvLegacy<HKHIP_IQ4_NL> {};
+template <> struct MvFmt<HKHIP_MXFP4> : MvLegacy<HKHIP_MXFP4> {};
 template <> struct MvFmt<HKHIP_Q4_0> : MvLegacy<HKHIP_Q4_0> {};
 template <> struct MvFmt<HKHIP_Q4_1> : MvLegacy<HKHIP_Q4_1> {};
 template <> struct MvFmt<HKHIP_Q5_0> : MvLegacy<HKHIP_Q5_0> {};
@@ -1205,13 +1292,13 @@ __host__ __device__ constexpr int mvr_rows(int nt, int c) { return nt == 1 ? (c 
 __host__ __device__ constexpr int mvr_cmax(int t, int nt) {
     return t == HKHIP_Q4_K || t == HKHIP_IQ4_XS ? (nt == 1 ? 4 : nt == 8 ? 1 : 2)
          : t == HKHIP_Q5_K ? (nt == 1 ? 2 : 1)
-         : t == HKHIP_Q6_K ? (nt == 1 ? 4 : nt == 2 ? 2 : 1)
+         : t == HKHIP_Q6_K || t == HKHIP_Q3_K || t == HKHIP_Q2_K ? (nt == 1 ? 4 : nt == 2 ? 2 : 1)
                            : (nt == 1 ? 8 : nt == 8 ? 2 : 4);
 }
 // Waves per workgroup: MVR_NWAVES (a budget of 256 registers per lane), or 4 (512) for the
 // variants that need more.
 __host__ __device__ constexpr int mvr_nw(int t, int nt, int c) {
-    return ((t == HKHIP_Q6_K || t == HKHIP_Q5_K) && nt * c >= 4) ||
+    return ((t == HKHIP_Q6_K || t == HKHIP_Q5_K || t == HKHIP_Q3_K || t == HKHIP_Q2_K) && nt * c >= 4) ||
                    ((t == HKHIP_Q4_K || t == HKHIP_IQ4_XS) && nt * c >= 8 && nt < 8) ||
                    (legacy32(t) && c >= 4 && nt * c >= 8)
                ? 4
@@ -1318,6 +1405,15 @@ extern template mv_kernel_t mvs_pick<HKHIP_Q5_0>(int, int);
 extern template mv_kernel_t pick<HKHIP_Q5_1>(int);
 extern template mv_kernel_t mvr_pick<HKHIP_Q5_1>(int, int, int, bool);
 extern template mv_kernel_t mvs_pick<HKHIP_Q5_1>(int, int);
+extern template mv_kernel_t pick<HKHIP_Q3_K>(int);
+extern template mv_kernel_t mvr_pick<HKHIP_Q3_K>(int, int, int, bool);
+extern template mv_kernel_t mvs_pick<HKHIP_Q3_K>(int, int);
+extern template mv_kernel_t pick<HKHIP_Q2_K>(int);
+extern template mv_kernel_t mvr_pick<HKHIP_Q2_K>(int, int, int, bool);
+extern template mv_kernel_t mvs_pick<HKHIP_Q2_K>(int, int);
+extern template mv_kernel_t pick<HKHIP_MXFP4>(int);
+extern template mv_kernel_t mvr_pick<HKHIP_MXFP4>(int, int, int, bool);
+extern template mv_kernel_t mvs_pick<HKHIP_MXFP4>(int, int);
 #endif
 
 } // namespace hkhip

@@ -51,6 +51,7 @@ template <> struct Fmt<HKHIP_Q8_0> {
 template <> struct Fmt<HKHIP_IQ4_NL> {
     static constexpr uint32_t RB = 128, W16 = 4, W4 = 0, WSB = 1024, DAB = 32;
 };
+template <> struct Fmt<HKHIP_MXFP4> : Fmt<HKHIP_IQ4_NL> {};
 // Q4_0..Q5_1: side data per row and step: d (16 B) and m (16 B) as one 1-KB load per wave (lanes
 // 32-63 take m), the fifth-bit words (32 B) as a second.
 template <int T> struct Fmt4 {
@@ -453,7 +454,7 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
                 const uint4 s16 = *reinterpret_cast<const uint4 *>(&S.ws[wave][16 * j]);
                 const uint32_t sw4[4] = {s16.x, s16.y, s16.z, s16.w};
 #pragma unroll
-                for (int c = 0; c < 8; c++) dw[c] = f16_bits_to_f32((sw4[c / 2] >> (16 * (c & 1))) & 0xFFFF);
+                for (int c = 0; c < 8; c++) dw[c] = block_scale<T>((sw4[c / 2] >> (16 * (c & 1))) & 0xFFFF);
             }
             load_a(0);
 #pragma unroll
@@ -559,6 +560,13 @@ hipError_t launch_cfg(const MxArgs &a0, hipStream_t s) {
     return hipGetLastError();
 }
 
+// IQ4_NL and MXFP4. Few row blocks (4096 x 14336: 139 vs 234 us): two K slices instead of 256-row tiles.
+template <int T> hipError_t launch_codebook(const MxArgs &a, hipStream_t s, uint32_t b82, uint32_t b42) {
+    if (b82 >= 224) return launch_cfg<T, 8, 2, 2>(a, s);
+    if (b42 >= 128 && a.cols >= 1024) return launch_cfg<T, 4, 2, 2, 2>(a, s);
+    return launch_cfg<T, 4, 1, 2>(a, s);
+}
+
 // Q4_0..Q5_1: IQ4_NL's tile choice (same quant bytes per block).
 template <int T> hipError_t launch_low4(const MxArgs &a, hipStream_t s, uint32_t b82, uint32_t b42) {
     if (b82 >= 224) return launch_cfg<T, 8, 2, 2>(a, s);
@@ -622,11 +630,8 @@ hipError_t launch_mmx(int t, const uint8_t *w, uint32_t rows, uint32_t cols, con
         return mx::launch_cfg<HKHIP_Q6_K, 4, 1, 2>(a, s);
     case HKHIP_Q8_0:
         return mx::launch_cfg<HKHIP_Q8_0, 4, 1, 2>(a, s);
-    case HKHIP_IQ4_NL:
-        // Few row blocks (4096 x 14336: 139 vs 234 us): two K slices instead of 256-row tiles.
-        if (blocks(8, 2) >= 224) return mx::launch_cfg<HKHIP_IQ4_NL, 8, 2, 2>(a, s);
-        if (blocks(4, 2) >= 128 && cols >= 1024) return mx::launch_cfg<HKHIP_IQ4_NL, 4, 2, 2, 2>(a, s);
-        return mx::launch_cfg<HKHIP_IQ4_NL, 4, 1, 2>(a, s);
+    case HKHIP_IQ4_NL: return mx::launch_codebook<HKHIP_IQ4_NL>(a, s, blocks(8, 2), blocks(4, 2));
+    case HKHIP_MXFP4: return mx::launch_codebook<HKHIP_MXFP4>(a, s, blocks(8, 2), blocks(4, 2));
     case HKHIP_Q4_0: return mx::launch_low4<HKHIP_Q4_0>(a, s, blocks(8, 2), blocks(4, 2));
     case HKHIP_Q4_1: return mx::launch_low4<HKHIP_Q4_1>(a, s, blocks(8, 2), blocks(4, 2));
     case HKHIP_Q5_0: return mx::launch_low4<HKHIP_Q5_0>(a, s, blocks(8, 2), blocks(4, 2));

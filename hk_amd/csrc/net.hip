@@ -1592,7 +1592,7 @@ int product(hkhip_net *net, uint32_t n, const hkhip_mat *mats, uint32_t nparts, 
             return hkhip_matvec_parts(eng, mats, nparts, nullptr, net->xq, n, ys, biases, mode);
         }
         if (norm) {
-            const int rc = hkhip_matvec_parts_rmsnorm(eng, mats, nparts, xin, norm, net->cfg.rms_eps, n, ys, biases, mode);
+            const int rc = matvec_parts_rmsnorm(eng, mats, nparts, xin, norm, net->cfg.rms_eps, n, ys, biases, mode, true);
             if (rc != HKHIP_E_UNSUPPORTED_SHAPE) return rc;
             hipLaunchKernelGGL(rmsnorm_kernel, dim3(n), dim3(256), 0, eng->cur, xin, norm, net->xb, cols, net->cfg.rms_eps);
             NET_TRY(hipGetLastError(), "rmsnorm");

@@ -61,6 +61,21 @@ __global__ void repack_kernel(int t, const uint8_t *__restrict__ src, uint8_t *_
         scales[b] = uint16_t(s[0] | (s[1] << 8));
         uint8_t *q = dst + b * 16;
         for (int j = 0; j < 16; j++) q[j] = s[2 + j];
+    } else if (t == HKHIP_MXFP4) { // e, qs[16]; the scale as the top half of its f32 (e8m0Half: 2^(e - 128))
+        const uint8_t *s = src + b * 17;
+        scales[b] = uint16_t((s[0] < 2 ? (0x00200000u << s[0]) : uint32_t(s[0] - 1) << 23) >> 16);
+        uint8_t *q = dst + b * 16;
+        for (int j = 0; j < 16; j++) q[j] = s[1 + j];
+    } else if (t == HKHIP_Q3_K) { // hmask[32] qs[64] | scales[12] d
+        const uint8_t *s = src + b * 110;
+        uint8_t *q = dst + b * 96, *side = dst + scale_off + b * 16;
+        for (int j = 0; j < 96; j++) q[j] = s[j];
+        for (int j = 0; j < 16; j++) side[j] = j < 14 ? s[96 + j] : 0;
+    } else if (t == HKHIP_Q2_K) { // scales[16] | qs[64] | d dmin
+        const uint8_t *s = src + b * 84;
+        uint8_t *q = dst + b * 64, *side = dst + scale_off + b * 20;
+        for (int j = 0; j < 64; j++) q[j] = s[16 + j];
+        for (int j = 0; j < 20; j++) side[j] = s[j < 16 ? j : 64 + j];
     } else { // Q6_K: ql[128] qh[64] scales[16] d
         const uint8_t *s = src + b * 210;
         scales[b] = uint16_t(s[208] | (s[209] << 8));
@@ -153,6 +168,27 @@ __global__ void dequant_kernel(int t, const uint8_t *__restrict__ w, uint32_t co
         uint32_t nib = hi ? (q >> 4) : (q & 0x0F);
         if (five) nib += ((blk[16 + l] >> (2 * chunk + hi)) & 1) * 16;
         v = d1 * (float)nib - m1;
+    } else if (t == HKHIP_MXFP4) { // dequant.zig:506-519
+        const uint64_t b = r * (cols / 32) + c / 32;
+        const uint32_t j = c % 32;
+        const uint8_t byte = w[b * 16 + (j & 15)];
+        const int8_t q = (int8_t)(fp4_lookup4(j < 16 ? (byte & 0x0F) : (byte >> 4)) & 0xFF);
+        v = (float)q * block_scale<HKHIP_MXFP4>(scales[b]);
+    } else if (t == HKHIP_Q2_K || t == HKHIP_Q3_K) { // dequant.zig:80-112, 114-165
+        const uint64_t b = r * (cols / 256) + c / 256;
+        const uint32_t e = c % 256, n = e / 128, it = (e % 128) / 32, l = e % 32, g = e / 16; // group g = 8n + 2it + l/16
+        if (t == HKHIP_Q2_K) {
+            const uint8_t *side = w + scale_off + b * 20;
+            const float dl = f16_bits_to_f32(side[16] | (side[17] << 8)) * (float)(side[g] & 0x0F);
+            const float ml = f16_bits_to_f32(side[18] | (side[19] << 8)) * (float)(side[g] >> 4);
+            v = dl * (float)((w[b * 64 + 32 * n + l] >> (2 * it)) & 3) - ml;
+        } else {
+            const uint8_t *side = w + scale_off + b * 16, *blk = w + b * 96;
+            const uint32_t lo = (side[g % 8] >> (g < 8 ? 0 : 4)) & 0x0F, hi = (side[8 + g % 4] >> (2 * (g / 4))) & 3;
+            const float dl = f16_bits_to_f32(side[12] | (side[13] << 8)) * (float)(int(lo | (hi << 4)) - 32);
+            const int q = int((blk[32 + 32 * n + l] >> (2 * it)) & 3) - ((blk[l] >> (4 * n + it)) & 1 ? 0 : 4);
+            v = dl * (float)q;
+        }
     } else { // Q6_K
         uint64_t b = r * (cols / 256) + c / 256;
         const uint8_t *blk = w + b * 208;

@@ -40,9 +40,11 @@ extern "C" {
 #define HKHIP_Q6_K 0x44
 #define HKHIP_IQ4_NL 0x55
 #define HKHIP_IQ4_XS 0x56
-/* Formats whose products decode the weights to floats first, hk's "exact fallback" (vecdot.zig
- * dotCanonK / dotCanonLegacy / dotGeneric): upload, bit-exact decode and products (1..8 tokens per
- * decode pass; longer inputs in passes), no MFMA GEMM (src/format.zig:71-93). */
+/* Formats whose products hk computes on weights decoded to floats first, its "exact fallback"
+ * (vecdot.zig dotCanonK / dotCanonLegacy / dotGeneric; src/format.zig:71-93): upload, bit-exact decode
+ * and products. Q2_K, Q3_K and MXFP4 run on exact integer sums like the formats above (decode kernels
+ * and MFMA GEMM); the others decode to floats in the kernel (1..8 tokens per pass; longer inputs in
+ * passes). */
 #define HKHIP_Q2_K 0x40
 #define HKHIP_Q3_K 0x41
 #define HKHIP_IQ1_S 0x50

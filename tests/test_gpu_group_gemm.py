@@ -1,0 +1,107 @@
+"""The prefill GEMM of the formats whose group scales fold into int8 weights (mmg.hip), at the
+edges of its tiles, against the products in float64 from the oracle's decoders and quantizer."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from hk_amd import formats as F
+from hk_amd import synth
+from hk_amd.engine import ACCUMULATE, SILU_MUL, STORE
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_cuda():
+    import torch
+
+    assert torch.cuda.is_available(), "GPU tests need a visible MI355X"
+    return torch
+
+
+@pytest.fixture(scope="module")
+def eng(torch_cuda):
+    from hk_amd import Engine
+
+    e = Engine(0)
+    e.set_stream(torch_cuda.cuda.current_stream().cuda_stream)
+    yield e
+    e.close()
+
+
+def products64(t, raw, m, k, x):
+    """(y, a bound on the f32 summation's error) of W times the quantized x, in float64: the exact
+    integers' scaled sums add k / 32 (k / 256) terms and scale each with at most 3 roundings, so they are
+    within (terms + 4) * 2^-23 of the sum of the terms' magnitudes."""
+    w = np.stack([O.dequantize(t, raw[r], k) for r in range(m)]).astype(np.float64)
+    kind = F.ACT_KIND[t]
+    el = 32 if kind == F.ACT_A8 else 256
+    a = np.empty(x.shape, np.float64)
+    for i, row in enumerate(x):
+        blk = (O.quantize_a8 if kind == F.ACT_A8 else O.quantize_q8k)(row).view(np.uint8).reshape(k // el, -1)
+        d = blk[:, :4].copy().view(np.float32).astype(np.float64)
+        qs = blk[:, 8:8 + el] if kind == F.ACT_A8 else blk[:, 4:4 + el]
+        a[i] = (d * qs.copy().view(np.int8)).reshape(-1)
+    return a @ w.T, (k // el + 4) * 2.0 ** -23 * (np.abs(a) @ np.abs(w).T)
+
+
+# (rows, K, tokens): each tile of the dispatch (by the rounds its grid takes), with whole and ragged
+# last rows and tokens, K of one super-block, and K slices that end at different super-blocks.
+SHAPES = [(32, 256, 9), (33, 256, 41), (70, 1280, 33), (96, 2304, 64), (1000, 768, 130), (4100, 1024, 65),
+          (8200, 512, 257), (14340, 256, 511)]
+
+
+@pytest.mark.parametrize("t", [F.Q3_K, F.Q2_K])
+@pytest.mark.parametrize("m,k,n", SHAPES)
+@pytest.mark.parametrize("mode", [STORE, ACCUMULATE, SILU_MUL])
+def test_group_gemm(eng, torch_cuda, t, m, k, n, mode):
+    torch = torch_cuda
+    m -= m % 2 if mode == SILU_MUL else 0
+    raw = synth.weights_np(t, m, k, seed=9100 + t + m)
+    x = synth.activations_np(n, k, seed=9101 + n, outliers=0.01)
+    want, bound = products64(t, raw, m, k, x)
+    bias = None if mode == SILU_MUL else np.linspace(-1, 1, m).astype(np.float32)
+    w = eng.upload(raw, t, m, k)
+    xq = torch.empty(eng.act_bytes(n, k), dtype=torch.uint8, device="cuda")
+    eng.qact(torch.from_numpy(x).cuda(), n, k, F.ACT_KIND[t], xq)
+    y0 = synth.activations_np(n, m // 2 if mode == SILU_MUL else m, seed=9102)
+    y = torch.from_numpy(y0.copy()).cuda()
+    eng.gemm(w, xq, y, n, bias=None if bias is None else torch.from_numpy(bias).cuda(), mode=mode)
+    got = y.cpu().numpy().astype(np.float64)
+    eng.free(w)
+    if mode == SILU_MUL:
+        g, u = want[:, 0::2], want[:, 1::2]
+        sig = 1.0 / (1.0 + np.exp(-g))
+        # d silu(g) u = (sig + g sig (1 - sig)) u dg + silu(g) du, and the f32 silu itself.
+        slope = np.abs(sig * (1.0 + g * (1.0 - sig)))
+        bound = slope * np.abs(u) * bound[:, 0::2] + np.abs(g * sig) * bound[:, 1::2] + 2.0 ** -20 * np.abs(g * sig * u)
+        want = g * sig * u
+    else:
+        want = want + bias
+        if mode == ACCUMULATE:
+            want = want + y0
+        bound = bound + 2.0 ** -22 * (np.abs(want) + np.abs(y0) + 1.0)
+    assert np.all(np.abs(got - want) <= bound + 1e-30)
+
+
+@pytest.mark.parametrize("n", [33, 70, 300])
+@pytest.mark.parametrize("m,k", [(40, 256), (300, 2048), (8200, 256)])
+def test_mxfp4_gemm(eng, torch_cuda, m, k, n):
+    """MXFP4's products from 25 tokens: the 32-weight GEMM on a power-of-two scale plane, the smallest
+    and largest exponents among them."""
+    torch = torch_cuda
+    raw = synth.weights_np(F.MXFP4, m, k, seed=9200 + m)
+    raw.reshape(-1, 17)[::37, 0] = 0
+    raw.reshape(-1, 17)[5::41, 0] = 1
+    raw.reshape(-1, 17)[7::43, 0] = 140
+    x = synth.activations_np(n, k, seed=9201 + n)
+    want, bound = products64(F.MXFP4, raw, m, k, x)
+    w = eng.upload(raw, F.MXFP4, m, k)
+    xq = torch.empty(eng.act_bytes(n, k), dtype=torch.uint8, device="cuda")
+    eng.qact(torch.from_numpy(x).cuda(), n, k, F.ACT_A8, xq)
+    y = torch.full((n, m), float("nan"), device="cuda")
+    eng.mm(w, xq, y, n)
+    assert np.all(np.abs(y.cpu().numpy() - want) <= bound + 1e-30)
+    eng.free(w)
