@@ -27,7 +27,11 @@
 // MFMA and 7 ns per MFMA plus 1.8 ns per VALU instruction: at 128 tokens per wave Q6_K's ~64 MFMAs and
 // ~740 VALU instructions per super-block are VALU-bound.
 // Measured at 512 tokens: Q3_K 14336 x 4096 30.6 ms (decode passes of 8 tokens on float-decoded
-// weights) -> 53 us, Q2_K 57 us (1050 TOPS).
+// weights) -> 53 us, Q2_K 57 us (1050 TOPS); Q6_K, against a tile that rebuilt its planes every 64
+// tokens with one wave per SIMD, 14336 x 4096 169 -> 82 us, 4096 x 14336 152 -> 105 us, at 100 tokens
+// 90 -> 44 us, 1024 x 4096 29.4 -> 15.9 us. (A three-slot ring with the barrier moved inside the step and
+// the planes built one super-block ahead was no faster, 109 -> 114 us at 4096 x 14336: neither the
+// barrier nor the loads' latency is what bounds it.)
 // MFMA roles: A = activations (tokens as M), B = weights (rows as N); output lane l holds row l%32
 // and tokens 8*(v/4) + 4*(l/32) + v%4.
 
@@ -476,7 +480,7 @@ template <int T> hipError_t launch_fmt(const MgArgs &a, hipStream_t s) {
 } // namespace mg
 
 bool mmg_supports(int t, uint32_t rows, uint32_t cols, uint32_t n) {
-    if (t != HKHIP_Q3_K && t != HKHIP_Q2_K) return false;
+    if (t != HKHIP_Q6_K && t != HKHIP_Q3_K && t != HKHIP_Q2_K) return false;
     if (cols % 256 != 0 || rows == 0 || n == 0) return false;
     // 32-bit per-lane byte offsets: quant plane, side plane and activations.
     const WLayout W = weight_layout(t, rows, cols);

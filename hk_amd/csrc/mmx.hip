@@ -1,14 +1,8 @@
-// Prefill GEMM for Q6_K and the 32-weight formats (Q8_0, IQ4_NL, Q4_0, Q4_1, Q5_0, Q5_1) on the
-// int8 MFMA units (K a multiple of 256).
+// Prefill GEMM for the 32-weight formats (Q8_0, IQ4_NL, MXFP4, Q4_0, Q4_1, Q5_0, Q5_1), Q5_K and
+// IQ4_XS on the int8 MFMA units (K a multiple of 256).
 //
-// Integer arithmetic as in hk's CPU kernels (src/quant/gemm.zig kernelK 180-236 for Q6_K,
-// kernelLegacy 131-176 for the 32-weight blocks):
-//  * Q6_K: per row r, token t and super-block b, y += d[r,b]*da[t,b] * I with the exact integer
-//    I = sum_g sc[r,b,g] * sum_{k in g} (q[r,k] - 32) * a[t,k] over the 16 groups of 16. The
-//    signed 8-bit group scale is folded into the weights, w = sc*(q - 32) in [-4096, 4096], and
-//    w is split into two int8 planes, 4*w = 256*H + L with H in [-63, 64] and L in [-128, 124].
-//    Each MFMA lane holds 16 weights of one group (one scale per lane and chunk). One int32
-//    chain per tile gives (H-sum << 8) + L-sum = 4*I, the reference's integer times four.
+// Integer arithmetic as in hk's CPU kernels (src/quant/gemm.zig kernelLegacy 131-176 for the
+// 32-weight blocks, kernelK 180-236 per sub-block for Q5_K and IQ4_XS):
 //  * 32-weight formats: y += (dw[r,c]*da[t,c]) * I_c per block c (I_c exact). One 32x32x32
 //    int8 MFMA yields the tile's I_c; then per output one multiply (dw*da), one convert and one
 //    fma. Q4_0 / Q5_0 weights enter as u - zp (kernelLegacy's acci - zp*s); Q4_1 / Q5_1 as u,
@@ -38,15 +32,12 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 // Per-format geometry of one super-block step (256 weights of 32 rows = one wave's share).
 template <int T> struct Fmt;
-template <> struct Fmt<HKHIP_Q6_K> {
-    static constexpr uint32_t RB = 208;  // quant-plane bytes per row and step
-    static constexpr uint32_t W16 = 6;   // 1-KB direct loads per wave
-    static constexpr uint32_t W4 = 2;    // 256-B direct loads (the rest)
-    static constexpr uint32_t WSB = 256; // scale bytes per wave (one dword per lane)
-    static constexpr uint32_t DAB = 4;   // activation-scale bytes per token and step
-};
 template <> struct Fmt<HKHIP_Q8_0> {
-    static constexpr uint32_t RB = 256, W16 = 8, W4 = 0, WSB = 1024, DAB = 32;
+    static constexpr uint32_t RB = 256;   // quant-plane bytes per row and step
+    static constexpr uint32_t W16 = 8;    // 1-KB direct loads per wave
+    static constexpr uint32_t W4 = 0;     // 256-B direct loads (the rest)
+    static constexpr uint32_t WSB = 1024; // scale bytes per wave
+    static constexpr uint32_t DAB = 32;   // activation-scale bytes per token and step
 };
 template <> struct Fmt<HKHIP_IQ4_NL> {
     static constexpr uint32_t RB = 128, W16 = 4, W4 = 0, WSB = 1024, DAB = 32;
@@ -62,7 +53,7 @@ template <int T> struct Fmt4 {
 template <> struct Fmt<HKHIP_IQ4_XS> {
     static constexpr uint32_t RB = 128, W16 = 4, W4 = 0, WSB = 256, DAB = 4;
 };
-// Q5_K: hk's 176-B blocks as they are (header, qh[32], qs[128]); rows unswizzled like Q6_K's.
+// Q5_K: hk's 176-B blocks as they are (header, qh[32], qs[128]); rows unswizzled.
 template <> struct Fmt<HKHIP_Q5_K> {
     static constexpr uint32_t RB = 176, W16 = 5, W4 = 2, WSB = 16, DAB = 4;
 };
@@ -77,9 +68,9 @@ template <int T, int TOK, int NW, bool MF = true> struct MxSlot {
     int8_t a[TOK * 256];                     // chunk c of token t at c ^ (t & 15)
     uint8_t w[NW][32 * Fmt<T>::RB];          // per wave, its 32 rows' bytes of the step
     uint8_t ws[NW][Fmt<T>::WSB];             // per wave, the rows' f16 scales of the step
-    // Activation scales: Q6_K per token (wave m fills tokens 64m..64m+63); A8 per block and token,
+    // Activation scales: Q8K per token (wave m fills tokens 64m..64m+63); A8 per block and token,
     // block-major ([8][TOK]), so that four consecutive tokens' scales are one 16-byte read.
-    float da[T == HKHIP_Q6_K || T == HKHIP_IQ4_XS || T == HKHIP_Q5_K ? 64 * NW : 8 * TOK];
+    float da[T == HKHIP_IQ4_XS || T == HKHIP_Q5_K ? 64 * NW : 8 * TOK];
     // Q5_K: each sub-block's d_a * bsum32; Q4_1 / Q5_1 without MF: the blocks' d_a * s (f32
     // bits, [8][TOK] as da).
     uint32_t sa[T == HKHIP_Q5_K || (has_m(T) && !MF) ? 8 * TOK : 1];
@@ -113,11 +104,10 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
     using F = Fmt<T>;
     constexpr bool mf = has_m(T) && KS == 1; // offset term on MFMAs
     using Slot = MxSlot<T, TOK, NW, KS == 1>;
-    constexpr bool q6 = (T == HKHIP_Q6_K);
     constexpr bool xs = (T == HKHIP_IQ4_XS);
     constexpr bool k5 = (T == HKHIP_Q5_K);
-    constexpr bool kqa = q6 || xs || k5; // Q8K activations: one scale per token and super-block
-    constexpr bool unswz = q6 || k5;     // rows not a power of two of pieces: no swizzle, word tail
+    constexpr bool kqa = xs || k5; // Q8K activations: one scale per token and super-block
+    constexpr bool unswz = k5;           // rows not a power of two of pieces: no swizzle, word tail
     constexpr uint32_t DBS = 8 * TOK / (64 * NW); // Q5_K: bsum-pair loads per wave
     static_assert(NB == 2 || NB == 3, "ring depth");
     static_assert(kqa ? TOK <= 64 * NW : (8 * TOK) % (64 * NW) == 0, "token scales per wave");
@@ -166,7 +156,7 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
                              (k5 ? DBS : 0);
     // Weights: 16-byte piece P = 64*i + lane of the wave's area is row P/(RB/16), piece P%(RB/16);
     // rows of 256 or 128 bytes are swizzled (piece c of row r at c ^ (r & 15), resp. r & 7) so
-    // the 32 rows one operand read covers hit distinct banks. Q6_K's 208-byte rows need no
+    // the 32 rows one operand read covers hit distinct banks. Q5_K's 176-byte rows need no
     // swizzle; its last 512 bytes go as words.
     constexpr uint32_t PPR = F::RB / 16;
     uint32_t woff[F::W16 + F::W4];
@@ -185,15 +175,14 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
             woff[F::W16 + i] = rr * nsb * F::RB + 4 * (Wd % (F::RB / 4));
         }
     }
-    // Scales: Q6_K one f16 per row and step (the aligned dword holding it); the blocks' eight
-    // f16 (16 bytes) per row and step otherwise. Lanes 32-63 repeat lanes 0-31.
+    // Scales: the blocks' eight f16 (16 bytes) per row and step. Lanes 32-63 repeat lanes 0-31.
     // Q4_0..Q5_1 (side plane per row: d[nbr], m[nbr], qh[nbr]): lanes 32-63 load m, and the
     // fifth-bit words of blocks 0-3 (lanes 0-31) and 4-7 (lanes 32-63) go as a second load.
     const uint32_t srow = clamp_row(r0 + 32 * wave + j);
     constexpr bool low4 = has_m(T) || has_qh(T) || zero_point(T) != 0;
     const SideGeom G = side_geom(T, K / 32);
     const uint32_t sidebase = srow * G.stride;
-    const uint32_t sbase = q6 ? srow * nsb : !low4 ? srow * G.stride : sidebase + (h && has_m(T) ? G.m_off : 0);
+    const uint32_t sbase = !low4 ? srow * G.stride : sidebase + (h && has_m(T) ? G.m_off : 0);
     const uint32_t qhbase = sidebase + G.qh_off + 16 * h;
     const uint32_t xsoff = clamp_row(r0 + 32 * wave + lane / 2) * nsb * 8 + 4 * (lane % 2);
     // Q5_K d_a * bsum32: load i of wave m covers entries 64*(DBS*m + i) .. of [8][TOK]: sub-block
@@ -214,7 +203,7 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
         const uint32_t c = (lane % 16) ^ (tl & 15);
         aoff[i] = clamp_tok(t0 + tl) * K + 16 * c;
     }
-    // Token scales: Q6_K lane L of wave m loads token 64m + L's; A8 load i of wave m covers the
+    // Token scales: Q8K lane L of wave m loads token 64m + L's; A8 load i of wave m covers the
     // 64 entries 64*(DAL*m + i) .. of the [8][TOK] array: block e / TOK, token e % TOK.
     uint32_t doff[DAL];
 #pragma unroll
@@ -247,10 +236,7 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
 #pragma unroll
         for (uint32_t i = 0; i < F::W4; i++) load_lds4(gw + woff[F::W16 + i], &S.w[wave][1024 * F::W16 + 256 * i]);
         const uint8_t *gd = reinterpret_cast<const uint8_t *>(a.ad);
-        if constexpr (q6) {
-            load_lds4(a.ws + (((sbase + sb) >> 1) << 2), &S.ws[wave][0]);
-            load_lds4(gd + doff[0] + 4 * sb, &S.da[64 * wave]);
-        } else if constexpr (xs) {
+        if constexpr (xs) {
             load_lds4(a.ws + xsoff + 8 * sb, &S.ws[wave][0]);
             load_lds4(gd + doff[0] + 4 * sb, &S.da[64 * wave]);
         } else if constexpr (k5) {
@@ -309,63 +295,7 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
                 av[c] = *reinterpret_cast<const v4i *>(abase + 32 * t * 256 + 16 * ((2 * c + h) ^ sw));
         };
 
-        if constexpr (q6) {
-            // This lane's row half: group 2c + h of chunk c = 4n + p is ql bytes 64n + 32(p&1) +
-            // 16h.. (nibble p>>1), qh bytes 128 + 32n + 16h.. (bits 2p), scale byte 192 + 8n + 2p + h
-            // (dequant.zig's Q6_K order).
-            const uint8_t *blk = &S.w[wave][208 * j];
-            uint4 ql[2][2], qh[2];
-#pragma unroll
-            for (int n = 0; n < 2; n++) {
-#pragma unroll
-                for (int pp = 0; pp < 2; pp++) ql[n][pp] = *reinterpret_cast<const uint4 *>(blk + 64 * n + 32 * pp + 16 * h);
-                qh[n] = *reinterpret_cast<const uint4 *>(blk + 128 + 32 * n + 16 * h);
-            }
-            const uint4 scw = *reinterpret_cast<const uint4 *>(blk + 192);
-            const uint32_t scs[4] = {scw.x, scw.y, scw.z, scw.w};
-            const uint32_t dword = *reinterpret_cast<const uint32_t *>(&S.ws[wave][4 * j]);
-            const float d = f16_bits_to_f32(((sbase + sb) & 1) ? dword >> 16 : dword & 0xFFFF);
-            // Planes H, L of the group-scaled weights (4*w = 256*H + L).
-            v4i P[2][8];
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const int n = c / 4, p = c % 4;
-                const uint32_t sbyte = 8 * n + 2 * p + h;
-                const int sc = int(int8_t((scs[sbyte / 4] >> (8 * (sbyte % 4))) & 0xFF));
-                const uint32_t m = q6k_m(sc), k = q6k_k(sc);
-                const uint32_t qlw[4] = {ql[n][p & 1].x, ql[n][p & 1].y, ql[n][p & 1].z, ql[n][p & 1].w};
-                const uint32_t qhw[4] = {qh[n].x, qh[n].y, qh[n].z, qh[n].w};
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t q = ((qlw[i] >> (4 * (p >> 1))) & 0x0F0F0F0Fu) | (((qhw[i] >> (2 * p)) & 0x03030303u) << 4);
-                    int hp, lp;
-                    q6k_planes(q, m, k, hp, lp);
-                    P[0][c][i] = hp;
-                    P[1][c][i] = lp;
-                }
-            }
-            const float d4 = 0.25f * d;
-            load_a(0);
-#pragma unroll
-            for (int t = 0; t < TT; t++) {
-                v16i sacc = {};
-#pragma unroll
-                for (int c = 0; c < 8; c++) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[c], P[0][c], sacc, 0, 0, 0);
-#pragma unroll
-                for (int v = 0; v < 16; v++) sacc[v] <<= 8;
-#pragma unroll
-                for (int c = 0; c < 8; c++) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[c], P[1][c], sacc, 0, 0, 0);
-                if (t + 1 < TT) load_a(t + 1);
-                const float4 *dap = reinterpret_cast<const float4 *>(&S.da[32 * t + 4 * h]);
-#pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const float4 dv = dap[2 * g];
-                    const float ds[4] = {dv.x, dv.y, dv.z, dv.w};
-#pragma unroll
-                    for (int e = 0; e < 4; e++) acc[t][4 * g + e] = fmaf((float)sacc[4 * g + e], d4 * ds[e], acc[t][4 * g + e]);
-                }
-            }
-        } else {
+        {
             // Block c of this lane's row: its 16-byte piece (Q8_0: bytes 16h.. of the block;
             // IQ4_NL: the block's 16 bytes, low nibbles for h = 0, high for h = 1).
             const uint8_t *blk = &S.w[wave][F::RB * j];
@@ -591,7 +521,7 @@ template <int T> hipError_t launch_low4(const MxArgs &a, hipStream_t s, uint32_t
 } // namespace mx
 
 bool mmx_supports(int t, uint32_t rows, uint32_t cols, uint32_t n) {
-    if (t != HKHIP_Q6_K && t != HKHIP_IQ4_XS && t != HKHIP_Q5_K && !legacy32(t)) return false;
+    if (t != HKHIP_IQ4_XS && t != HKHIP_Q5_K && !legacy32(t)) return false;
     if (cols % 256 != 0 || rows == 0 || n == 0) return false;
     // 32-bit per-lane byte offsets: quant plane, scale plane and activations.
     const WLayout W = weight_layout(t, rows, cols);
@@ -603,15 +533,15 @@ hipError_t launch_mmx(int t, const uint8_t *w, uint32_t rows, uint32_t cols, con
     if (!mmx_supports(t, rows, cols, n)) return hipErrorInvalidValue;
     const WLayout W = weight_layout(t, rows, cols);
     const ActLayout A = act_layout(n, cols);
-    const bool q6 = act_kind(t) == HKHIP_ACT_Q8K; // Q6_K, IQ4_XS
+    const bool kq = act_kind(t) == HKHIP_ACT_Q8K; // Q5_K, IQ4_XS
     mx::MxArgs a{};
     a.w = w;
     a.ws = w + W.scale_off;
     a.rows = rows;
     a.cols = cols;
     a.n = n;
-    a.aqs = reinterpret_cast<const int8_t *>(xq + (q6 ? A.k_qs : A.a8_qs));
-    a.ad = reinterpret_cast<const float *>(xq + (q6 ? A.k_d : A.a8_d));
+    a.aqs = reinterpret_cast<const int8_t *>(xq + (kq ? A.k_qs : A.a8_qs));
+    a.ad = reinterpret_cast<const float *>(xq + (kq ? A.k_d : A.a8_d));
     a.ads = reinterpret_cast<const float *>(xq + A.a8_ds);
     a.adsb = xq + A.a8_dsb;
     a.adb = reinterpret_cast<const float *>(xq + A.k_db);
@@ -625,9 +555,6 @@ hipError_t launch_mmx(int t, const uint8_t *w, uint32_t rows, uint32_t cols, con
         return ((rows + 32 * nw - 1) / (32 * nw)) * ((n + 32 * tt - 1) / (32 * tt));
     };
     switch (t) {
-    case HKHIP_Q6_K:
-        if (blocks(4, 2) >= 192) return mx::launch_cfg<HKHIP_Q6_K, 4, 2, 2>(a, s);
-        return mx::launch_cfg<HKHIP_Q6_K, 4, 1, 2>(a, s);
     case HKHIP_Q8_0:
         return mx::launch_cfg<HKHIP_Q8_0, 4, 1, 2>(a, s);
     case HKHIP_IQ4_NL: return mx::launch_codebook<HKHIP_IQ4_NL>(a, s, blocks(8, 2), blocks(4, 2));

@@ -53,7 +53,7 @@ SHAPES = [(32, 256, 9), (33, 256, 41), (70, 1280, 33), (96, 2304, 64), (1000, 76
           (8200, 512, 257), (14340, 256, 511)]
 
 
-@pytest.mark.parametrize("t", [F.Q3_K, F.Q2_K])
+@pytest.mark.parametrize("t", [F.Q6_K, F.Q3_K, F.Q2_K])
 @pytest.mark.parametrize("m,k,n", SHAPES)
 @pytest.mark.parametrize("mode", [STORE, ACCUMULATE, SILU_MUL])
 def test_group_gemm(eng, torch_cuda, t, m, k, n, mode):
