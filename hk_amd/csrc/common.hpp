@@ -166,8 +166,8 @@ inline WLayout weight_layout(int t, uint32_t rows, uint32_t cols) {
 //         range of one super-block is contiguous -- the token-side operand of the Q4_1 / Q5_1
 //         GEMM's offset term, which runs on bf16 MFMAs,
 //   k_qs  [n][k] i8, k_d  [n][k/256] f32, k_bs [n][k/16] i16,
-//   k_db  [n][k/32] f32: d * (f32)(bsum of the 32 values of each sub-block), the Q5_K GEMM's
-//         min-term operand,
+//   k_db  [n][k/32] f32: not written (its space stays, so that a buffer's size, and with it what
+//         hkhip_mm_noalloc's fixed buffer takes, does not change),
 //   k_mb  [n][k/256][16] bf16: per super-block, its 8 sub-blocks' 32-value sums as exact bf16
 //         integers, bsum32 = 64*u + v with v in [0, 63]: 64*u for the 8 sub-blocks, then v --
 //         the token-side operand of the GEMM's integer min term, precomputed once
@@ -337,6 +337,7 @@ hipError_t launch_mmvq_parts_norm(int t, const MvPartDesc *parts, int nparts, ui
                                   hipStream_t s);
 hipError_t launch_mmvq(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n,
                        float *y, const float *bias, int mode, hipStream_t s);
+// Prefill GEMM for large Q4_K and Q5_K matrices of at most two super-blocks a row.
 bool mm2_supports(int t, uint32_t rows, uint32_t cols, uint32_t n);
 // Small-batch MFMA product (Q4_K, 1..32 tokens): weights streamed like the decode kernels.
 bool mmsk_supports(int t, uint32_t rows, uint32_t cols, uint32_t n);
@@ -344,11 +345,11 @@ hipError_t launch_mmsk(int t, const uint8_t *w, uint32_t rows, uint32_t cols, co
                        float *y, const float *bias, int mode, hipStream_t s);
 hipError_t launch_mmsk_parts(int t, const MvPartDesc *parts, int nparts, uint32_t cols, const uint8_t *xq,
                              uint32_t n, int mode, hipStream_t s);
-// Prefill GEMM for Q6_K, Q3_K and Q2_K (cols a multiple of 256).
+// Prefill GEMM for Q4_K, Q5_K, Q6_K, Q3_K and Q2_K (cols a multiple of 256).
 bool mmg_supports(int t, uint32_t rows, uint32_t cols, uint32_t n);
 hipError_t launch_mmg(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n, float *y,
                       const float *bias, int mode, hipStream_t s);
-// Prefill GEMM for the 32-weight formats, Q5_K and IQ4_XS (cols a multiple of 256).
+// Prefill GEMM for the 32-weight formats and IQ4_XS (cols a multiple of 256).
 bool mmx_supports(int t, uint32_t rows, uint32_t cols, uint32_t n);
 hipError_t launch_mmx(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n, float *y,
                       const float *bias, int mode, hipStream_t s);

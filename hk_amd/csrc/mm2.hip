@@ -1,4 +1,7 @@
-// Prefill GEMM for Q4_K on the int8 MFMA units, split-plane form.
+// Prefill GEMM for Q4_K and Q5_K rows of one or two super-blocks on the int8 MFMA units, split-plane form:
+// there the output stores are a large part of the launch, and this tile stores each token tile beside
+// the next one's MFMAs (28672 x 512 at 512 tokens 27.7 us, against 29.9 on the tiles of mmg.hip, which
+// are faster from three super-blocks on: 14336 x 4096 83 -> 73 us).
 //
 // Per row r, token t and super-block b, hk's CPU kernel (src/quant/gemm.zig kernelK 180-236,
 // with the scale unpack of unpack.zig) computes
@@ -11,15 +14,10 @@
 //    bytes. Two int32 MFMA chains over the super-block's 256 weights give sum(sh*q*a) and
 //    sum(sl*q*a), combined exactly as (h << 3) + l -- the same integer as the reference's -- and
 //    applied with one f32 update per super-block.
-//  * min term: J = sum_s mn[s]*bsum32[s] is an integer below 2^22, and both factors are exact
-//    bf16 integers once bsum32 is written as 64*u + v (v in [0, 63]). The staged kernels run one
-//    32x32x16 bf16 MFMA with 64*u in its first 8 k and v in the other 8 (against mn in both),
-//    which yields J exactly in f32, and apply both terms in one update: y += da*(d*I - dmin*J).
-//    The large-tile kernel has no registers left for J's tile, so it folds the float scales into
-//    the operands instead, (-dmin*mn) x (da*bsum32), each split into three bf16 parts (their sum
-//    is the fp32 value to within 2^-24): a 32x32x16 MFMA pairs 8 sub-blocks of one token part
-//    (first 8 k) and another (last 8 k) with a row part, so three of them, (hi|mid) x h,
-//    (hi|mid) x m, (hi|lo) x (l|h), form every partial product down to 2^-24, accumulated in f32
+//  * min term: the float scales are folded into the operands, (-dmin*mn) x (da*bsum32), each split into
+//    three bf16 parts (their sum is the fp32 value to within 2^-24): a 32x32x16 MFMA pairs 8 sub-blocks
+//    of one token part (first 8 k) and another (last 8 k) with a row part, so three of them, (hi|mid) x
+//    h, (hi|mid) x m, (hi|lo) x (l|h), form every partial product down to 2^-24, accumulated in f32
 //    straight into the output tile.
 // Only the f32 summation order differs from the reference.
 //
@@ -49,31 +47,12 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 typedef short s2v __attribute__((ext_vector_type(2)));
 
-// Shapes: NW waves per workgroup (32 rows each), TT token tiles of 32 per wave, NB super-blocks
-// in flight; the workgroup covers 32*NW rows x 32*TT tokens. The large configuration amortizes
-// the weight unpack over 128 tokens; smaller ones keep small matrices spread over the CUs.
-// Everything a super-block needs arrives by direct global -> LDS loads into a ring of NB slots:
-//   a   token rows, 256 int8 each; 16-byte chunk c of token t sits at c ^ (t & 15) so the 32
-//       tokens one MFMA operand read covers hit distinct banks
-//   w   per wave, its 32 rows' 144-byte blocks back to back
-//   mb  per token, the min-term operand (k_mb of the activation buffer, 32 bytes)
-//   da  per token, the Q8K scale
-// Every wave issues the same loads (waves past the tokens load duplicates into their own spare
-// entries), so the in-order memory counter can be waited on with a constant.
-template <int TOK, int NW, int WB = 4608> struct Q2Slot {
-    int8_t a[TOK * 256];
-    uint8_t w[NW][WB]; // 32 rows x 144 (Q4_K) or 176 (Q5_K) bytes
-    uint32_t mb[NW * 32][8]; // token t at mb[t]; wave m's load fills tokens 32m..32m+31
-    float da[NW * 64];       // token t at da[t]; wave m's load fills tokens 64m..64m+63
-};
-
 struct Mm2Args {
     const uint8_t *w;
     uint32_t rows, cols, n;
     const int8_t *aqs;
     const float *ad;
     const int16_t *abs;
-    const uint8_t *amb; // k_mb: per token and super-block, 32 bytes (64*u, then v, as bf16)
     float *y;
     const float *bias;
     int mode;
@@ -131,29 +110,6 @@ __device__ __forceinline__ void min_term(v16f &acc, const uint32_t *tm, const Mi
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a12, B.b1, acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a12, B.b2, acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a3, B.b3, acc, 0, 0, 0);
-}
-
-// Row-side operand of the min term: the 8 sub-blocks' 6-bit mins (bytes of mnl, mnh) as bf16
-// integers, the same 8 values in both lane halves.
-__device__ __forceinline__ v8bf min_b(uint32_t mnl, uint32_t mnh) {
-    uint32_t w[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const uint32_t src = q < 2 ? mnl : mnh, sh = 16 * (q & 1);
-        const float e = (float)((src >> sh) & 0xFF), o = (float)((src >> (sh + 8)) & 0xFF);
-        w[q] = (__builtin_bit_cast(uint32_t, e) >> 16) | (__builtin_bit_cast(uint32_t, o) & 0xFFFF0000u);
-    }
-    return __builtin_bit_cast(v8bf, make_uint4(w[0], w[1], w[2], w[3]));
-}
-
-// J = sum_s mn[s] * bsum32[s] of a 32x32 tile, exact: tm holds this lane's token's 8 words
-// (64*u of the 8 sub-blocks in words 0-3, v in 4-7); lane half h supplies its half. `after` is
-// a value the caller computes just before: the operand is tied to it so that the MFMA is not
-// hoisted (with its result registers) ahead of the tile's other work.
-__device__ __forceinline__ v16f min_j(const uint32_t *tm, v8bf mn, uint32_t h, float after) {
-    uint4 w = *reinterpret_cast<const uint4 *>(tm + 4 * h);
-    asm volatile("" : "+v"(w.x) : "v"(after));
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, w), mn, v16f{}, 0, 0, 0);
 }
 
 // Q5_K: four 5-bit quants u (bytes; even bytes ev, odd od, as 16-bit lanes) times a factor e
@@ -435,278 +391,11 @@ __global__ __launch_bounds__(Q2_NW * 64, 2) void mm2_q4k_reg_kernel(Mm2Args a) {
 
 
 
-// KS > 1 splits K: the workgroup's waves form KS slices of NW waves; slice k takes super-blocks
-// k, k + KS, ... through a ring of its own, and the slices' partial tiles are added in LDS (in
-// slice order) at the end. For matrices too small to give every SIMD two waves otherwise.
-template <int NW, int TT, int NB, int KS = 1, int T = HKHIP_Q4_K>
-__global__ __launch_bounds__(NW * KS * 64, 2) void mm2_q4k_kernel(Mm2Args a) {
-    constexpr int ROWS = 32 * NW, TOK = 32 * TT;
-    // Q5_K: 176-byte rows (5 x 1 KB + 512 B per wave and step), the register tile's planes and
-    // a second exact integer, Jsc = sum sc*bsum32, for the 16*sum(sc*a) the planes' u - 16 removes.
-    constexpr bool k5 = (T == HKHIP_Q5_K);
-    constexpr uint32_t BB = k5 ? 176 : 144, PR = BB / 16, WR = BB / 4, W16 = k5 ? 5 : 4, QO = k5 ? 48 : 16;
-    using Slot = Q2Slot<TOK, NW, 32 * BB>;
-    static_assert(NB == 2 || NB == 3, "ring depth");
-    // The ring's slots are LDS objects of their own, and the loop below is unrolled over them.
-    __shared__ __attribute__((aligned(16))) Slot ring0[KS];
-    __shared__ __attribute__((aligned(16))) Slot ring1[KS];
-    __shared__ __attribute__((aligned(16))) Slot ring2[KS];
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
-    const uint32_t wall = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t ks = wall / NW, wave = wall % NW; // K slice, row wave within the slice
-    auto slot_at = [&](auto ic) -> Slot & {
-        constexpr int i = decltype(ic)::value;
-        if constexpr (i == 0)
-            return ring0[ks];
-        else if constexpr (i == 1)
-            return ring1[ks];
-        else
-            return ring2[ks];
-    };
-    const uint32_t h = lane >> 5, j = lane & 31;
-    const uint32_t K = a.cols, nsb = K / 256;
-
-    // Workgroup -> (row block, token block). The token blocks of one row block are consecutive
-    // workgroups on the same XCD (workgroups go round-robin over the 8 XCDs), so the rows they
-    // share are read from HBM once and then served by that XCD's L2.
-    uint32_t rb, tb;
-    {
-        const uint32_t i = blockIdx.x;
-        if (a.rblocks % 8 == 0) {
-            const uint32_t xcd = i % 8, k = i / 8;
-            rb = xcd * (a.rblocks / 8) + k / a.tblocks;
-            tb = k % a.tblocks;
-        } else {
-            rb = i / a.tblocks;
-            tb = i % a.tblocks;
-        }
-    }
-    const uint32_t r0 = rb * ROWS, t0 = tb * TOK;
-    const uint32_t myrow = r0 + 32 * wave + j;
-
-    // ---- the direct loads of one super-block into a slot (CPW per wave) ----
-    constexpr uint32_t TPW = TOK / NW; // token rows per wave
-    static_assert(TPW % 4 == 0, "token rows per wave");
-    constexpr uint32_t CPW = TPW / 4 + W16 + 2 + 1 + 1; // a + w + mb + da
-    // Weight bytes of this wave: 16-byte piece P (64*i + lane, i < 4) is byte 16*(P%9) of row
-    // P/9's block; the last 512 bytes (pieces 256..287) go as 4-byte words 1024 + 64*i + lane.
-    // Per-lane 32-bit byte offsets from uniform bases (mm2_supports checks that they fit).
-    uint32_t woff[W16 + 2];
-#pragma unroll
-    for (uint32_t i = 0; i < W16; i++) {
-        const uint32_t P = 64 * i + lane;
-        const uint32_t row = r0 + 32 * wave + P / PR, rr = row < a.rows ? row : a.rows - 1;
-        woff[i] = rr * nsb * BB + 16 * (P % PR);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const uint32_t Wd = 256 * W16 + 64 * i + lane; // 4-byte word index in the wave's area
-        const uint32_t row = r0 + 32 * wave + Wd / WR, rr = row < a.rows ? row : a.rows - 1;
-        woff[W16 + i] = rr * nsb * BB + 4 * (Wd % WR);
-    }
-    uint32_t aoff[TPW / 4];
-#pragma unroll
-    for (uint32_t i = 0; i < TPW / 4; i++) {
-        const uint32_t tl = TPW * wave + 4 * i + lane / 16;
-        const uint32_t c = (lane % 16) ^ (tl & 15);
-        const uint32_t tok = t0 + tl, tk = tok < a.n ? tok : a.n - 1;
-        aoff[i] = tk * K + 16 * c;
-    }
-    auto issue = [&](uint32_t sb, Slot &S) {
-        const int8_t *ga = a.aqs + 256 * sb;
-#pragma unroll
-        for (uint32_t i = 0; i < TPW / 4; i++) load_lds16(ga + aoff[i], &S.a[(TPW * wave + 4 * i) * 256]);
-        const uint8_t *gw = a.w + uint64_t(sb) * BB;
-#pragma unroll
-        for (uint32_t i = 0; i < W16; i++) load_lds16(gw + woff[i], &S.w[wave][1024 * i]);
-#pragma unroll
-        for (int i = 0; i < 2; i++) load_lds4(gw + woff[W16 + i], &S.w[wave][1024 * W16 + 256 * i]);
-        {
-            const uint32_t tl = 32 * wave + lane / 2, tok = t0 + (tl < TOK ? tl : 0);
-            const uint32_t tk = tok < a.n ? tok : a.n - 1;
-            load_lds16(a.amb + (uint64_t(tk) * nsb + sb) * 32 + 16 * (lane & 1), &S.mb[32 * wave][0]);
-        }
-        {
-            const uint32_t tl = 64 * wave + lane, tok = t0 + (tl < TOK ? tl : 0);
-            const uint32_t tk = tok < a.n ? tok : a.n - 1;
-            load_lds4(a.ad + uint64_t(tk) * nsb + sb, &S.da[64 * wave]);
-        }
-    };
-
-    v16f acc[TT];
-#pragma unroll
-    for (int t = 0; t < TT; t++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) acc[t][v] = 0.0f;
-
-    // Step j of slice ks is super-block ks + KS*j (loads past the end repeat the last one).
-    const uint32_t nst = (nsb + KS - 1) / KS;
-    auto sb_of = [&](uint32_t st) {
-        const uint32_t sb = ks + KS * st;
-        return sb < nsb ? sb : nsb - 1;
-    };
-
-    // Prologue: NB-1 super-blocks in flight.
-    issue(sb_of(0), slot_at(std::integral_constant<int, 0>{}));
-    if constexpr (NB == 3) issue(sb_of(1), slot_at(std::integral_constant<int, 1>{}));
-    // Wait for slot 0 (the loads of NB-2 later super-blocks may stay in flight).
-    __builtin_amdgcn_s_waitcnt((0x0F70 & ~0xF) | ((CPW * (NB - 2)) & 0xF) | (((CPW * (NB - 2)) >> 4) << 14));
-    __syncthreads();
-
-    // One super-block from slot IC while the one NB-1 ahead goes into slot (IC + NB-1) % NB.
-    auto step = [&](auto ic, uint32_t st) {
-        constexpr int I = decltype(ic)::value;
-        issue(sb_of(st + NB - 1), slot_at(std::integral_constant<int, (I + NB - 1) % NB>{}));
-        Slot &S = slot_at(ic);
-        if (KS == 1 || ks + KS * st < nsb) {
-            // Unpack this lane's row half (h) from LDS: header, then both planes of 8 sub-blocks.
-            const uint8_t *blk = &S.w[wave][BB * j];
-            const uint4 ch = *reinterpret_cast<const uint4 *>(blk);
-            uint4 cq[4], cx{};
-#pragma unroll
-            for (int p = 0; p < 4; p++) cq[p] = *reinterpret_cast<const uint4 *>(blk + QO + 32 * p + 16 * h);
-            if constexpr (k5) cx = *reinterpret_cast<const uint4 *>(blk + 16 + 16 * h);
-            // Scales: vecdot.zig:461-474 word form.
-            const uint32_t k1 = 0x3f3f3f3fu, k2 = 0x0f0f0f0fu, k3 = 0x03030303u;
-            const uint32_t scl = ch.y & k1, mnl = ch.z & k1;
-            const uint32_t sch = (ch.w & k2) | (((ch.y >> 6) & k3) << 4);
-            const uint32_t mnh = ((ch.w >> 4) & k2) | (((ch.z >> 6) & k3) << 4);
-            const float d = f16_bits_to_f32(ch.x & 0xFFFF), dmin = f16_bits_to_f32(ch.x >> 16);
-            v4i bhi[8], blo[8];
-#pragma unroll
-            for (int p = 0; p < 4; p++) {
-                const uint32_t se = (p < 2 ? scl >> (16 * p) : sch >> (16 * (p - 2))) & 0xFF;
-                const uint32_t so = (p < 2 ? scl >> (16 * p + 8) : sch >> (16 * (p - 2) + 8)) & 0xFF;
-                const uint32_t she = (se >> 3) * 0x00010001u, sle = (se & 7) * 0x00010001u;
-                const uint32_t sho = (so >> 3) * 0x00010001u, slo = (so & 7) * 0x00010001u;
-                const uint32_t qw[4] = {cq[p].x, cq[p].y, cq[p].z, cq[p].w};
-                const uint32_t xw[4] = {cx.x, cx.y, cx.z, cx.w};
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t ne = qw[i] & 0x0F0F0F0Fu, no = (qw[i] >> 4) & 0x0F0F0F0Fu;
-                    if constexpr (k5) {
-                        const uint32_t ue = ne | (((xw[i] >> (2 * p)) & 0x01010101u) << 4);
-                        const uint32_t uo = no | (((xw[i] >> (2 * p + 1)) & 0x01010101u) << 4);
-                        const uint32_t ee = ue & 0x00FF00FFu, eo = (ue >> 8) & 0x00FF00FFu;
-                        const uint32_t oe = uo & 0x00FF00FFu, oo = (uo >> 8) & 0x00FF00FFu;
-                        bhi[2 * p][i] = int(plane_c16(ee, eo, she, neg16(she)));
-                        blo[2 * p][i] = int(plane_c16(ee, eo, sle, neg16(sle)));
-                        bhi[2 * p + 1][i] = int(plane_c16(oe, oo, sho, neg16(sho)));
-                        blo[2 * p + 1][i] = int(plane_c16(oe, oo, slo, neg16(slo)));
-                    } else {
-                        bhi[2 * p][i] = int(mul_bytes(ne, she));
-                        blo[2 * p][i] = int(mul_bytes(ne, sle));
-                        bhi[2 * p + 1][i] = int(mul_bytes(no, sho));
-                        blo[2 * p + 1][i] = int(mul_bytes(no, slo));
-                    }
-                }
-            }
-            // Min-term operand of this lane's row.
-            const v8bf mB = min_b(mnl, mnh);
-            const v8bf sB = k5 ? min_b(scl, sch) : mB; // Q5_K: the scales as exact bf16 integers
-            const float ndmin = -dmin;
-
-            // A operand of tile t, sub-block s: token 32t + j, chunk 2s + h (swizzled).
-            const int8_t *abase = &S.a[j * 256];
-            const uint32_t sw = j & 15;
-            v4i av[8];
-            auto load_a = [&](int t) {
-#pragma unroll
-                for (int s = 0; s < 8; s++)
-                    av[s] = *reinterpret_cast<const v4i *>(abase + 32 * t * 256 + 16 * ((2 * s + h) ^ sw));
-            };
-            load_a(0);
-#pragma unroll
-            for (int t = 0; t < TT; t++) {
-                const v16f jt = min_j(S.mb[32 * t + j], mB, h, acc[t][15]);
-                v16f js = {};
-                if constexpr (k5) js = min_j(S.mb[32 * t + j], sB, h, jt[15]);
-                // One accumulator: the sh-plane chain, times 8, then the sl-plane chain on top.
-                v16i sacc = {};
-#pragma unroll
-                for (int s = 0; s < 8; s++) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[s], bhi[s], sacc, 0, 0, 0);
-#pragma unroll
-                for (int v = 0; v < 16; v++) sacc[v] <<= 3;
-#pragma unroll
-                for (int s = 0; s < 8; s++) sacc = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[s], blo[s], sacc, 0, 0, 0);
-                if (t + 1 < TT) load_a(t + 1);
-                // Token scales of this lane's 16 outputs: tokens 32t + 8g + 4h + (0..3).
-                const float4 *dap = reinterpret_cast<const float4 *>(&S.da[32 * t + 4 * h]);
-#pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const float4 dv = dap[2 * g];
-                    const float ds[4] = {dv.x, dv.y, dv.z, dv.w};
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const int v = 4 * g + e;
-                        const float iv = k5 ? fmaf(16.0f, js[v], (float)sacc[v]) : (float)sacc[v];
-                        acc[t][v] = fmaf(fmaf(iv, d, ndmin * jt[v]), ds[e], acc[t][v]);
-                    }
-                }
-            }
-        }
-        // The next super-block's slot has landed once at most NB-2 later issues are pending.
-        __builtin_amdgcn_s_waitcnt((0x0F70 & ~0xF) | ((CPW * (NB - 2)) & 0xF) | (((CPW * (NB - 2)) >> 4) << 14));
-        __syncthreads();
-    };
-    for (uint32_t st = 0; st < nst; st += NB) {
-        step(std::integral_constant<int, 0>{}, st);
-        if (st + 1 < nst) step(std::integral_constant<int, 1>{}, st + 1);
-        if constexpr (NB == 3)
-            if (st + 2 < nst) step(std::integral_constant<int, 2>{}, st + 2);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): no direct load still writing the ring
-    __syncthreads();                   // in any wave: the ring is free from here
-
-    if constexpr (KS > 1) {
-        // Slices 1.. leave their tiles in the ring; slice 0 adds them in order.
-        float *red = reinterpret_cast<float *>(&ring0[0]);
-        static_assert((KS - 1) * NW * TT * 16 * 64 * 4 <= KS * sizeof(Slot), "reduction space");
-        if (ks > 0) {
-#pragma unroll
-            for (int t = 0; t < TT; t++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) red[((((ks - 1) * NW + wave) * TT + t) * 16 + v) * 64 + lane] = acc[t][v];
-        }
-        __syncthreads();
-        if (ks == 0) {
-#pragma unroll
-            for (int k = 1; k < KS; k++)
-#pragma unroll
-                for (int t = 0; t < TT; t++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++) acc[t][v] += red[((((k - 1) * NW + wave) * TT + t) * 16 + v) * 64 + lane];
-        }
-        __syncthreads(); // the reduction area is read: the ring takes the output staging
-        if (ks > 0) return;
-    }
-
-    // ---- store: y[token][row], bias, accumulate ----
-    {
-        static_assert(NW * 4096 <= KS * sizeof(Slot), "output staging space");
-        float *st = reinterpret_cast<float *>(&ring0[0]) + 1024 * wave;
-        const float b = (a.bias && myrow < a.rows) ? a.bias[myrow] : 0.0f;
-        const uint32_t rw0 = r0 + 32 * wave;
-#pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const uint32_t tk0 = t0 + 32 * t;
-            if (a.wide && rw0 + 32 <= a.rows && tk0 + 32 <= a.n)
-                gemm_store_tile_wide(st, acc[t], b, a.y, a.rows, rw0, tk0, a.mode);
-            else
-                gemm_store_tile(acc[t], b, a.y, a.rows, a.n, myrow, tk0, a.mode);
-        }
-    }
-}
-
+// Two super-blocks at most, and enough 256 x 128 tiles for most CUs (a round of this tile costs as much
+// with fewer). The kernel's per-lane byte offsets into the activations are 32-bit.
 bool mm2_supports(int t, uint32_t rows, uint32_t cols, uint32_t n) {
-    // The kernels' per-lane byte offsets are 32-bit: weights rows*cols*9/16 bytes, activations
-    // n*cols bytes.
-    if (t == HKHIP_Q5_K) // the register tile and the 128-row ring tile, where they fill the GPU
-        return cols % 256 == 0 &&
-               (((rows + 255) / 256) * ((n + 127) / 128) >= 192 || ((rows + 127) / 128) * ((n + 63) / 64) >= 160) &&
-               uint64_t(rows) * (cols / 256) * 176 < (1ull << 32) && uint64_t(n) * cols < (1ull << 32);
-    return t == HKHIP_Q4_K && cols % 256 == 0 && rows > 0 && n > 0 &&
-           uint64_t(rows) * (cols / 256) * 144 < (1ull << 32) && uint64_t(n) * cols < (1ull << 32);
+    return (t == HKHIP_Q4_K || t == HKHIP_Q5_K) && cols > 0 && cols % 256 == 0 && cols <= 512 &&
+           ((rows + 255) / 256) * ((n + 127) / 128) >= 192 && uint64_t(n) * cols < (1ull << 32);
 }
 
 typedef void (*mm2_kernel_t)(Mm2Args);
@@ -727,18 +416,6 @@ static hipError_t launch_mm2_reg(const Mm2Args &a0, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int NW, int TT, int NB, int KS = 1, int T = HKHIP_Q4_K>
-static hipError_t launch_mm2_cfg(const Mm2Args &a0, hipStream_t s) {
-    const mm2_kernel_t k = mm2_q4k_kernel<NW, TT, NB, KS, T>;
-    static_assert(NB * KS * sizeof(Q2Slot<32 * TT, NW, T == HKHIP_Q5_K ? 5632 : 4608>) <= 160 * 1024, "LDS");
-    constexpr size_t lds = 0; // the ring is static
-    Mm2Args a = a0;
-    a.rblocks = (a.rows + 32 * NW - 1) / (32 * NW);
-    a.tblocks = (a.n + 32 * TT - 1) / (32 * TT);
-    hipLaunchKernelGGL(k, dim3(a.rblocks * a.tblocks), dim3(NW * KS * 64), lds, s, a);
-    return hipGetLastError();
-}
-
 hipError_t launch_mm2(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n, float *y,
                       const float *bias, int mode, hipStream_t s) {
     if (!mm2_supports(t, rows, cols, n)) return hipErrorInvalidValue;
@@ -751,32 +428,11 @@ hipError_t launch_mm2(int t, const uint8_t *w, uint32_t rows, uint32_t cols, con
     a.aqs = reinterpret_cast<const int8_t *>(xq + A.k_qs);
     a.ad = reinterpret_cast<const float *>(xq + A.k_d);
     a.abs = reinterpret_cast<const int16_t *>(xq + A.k_bs);
-    a.amb = xq + A.k_mb;
     a.y = y;
     a.bias = bias;
     a.mode = mode;
     a.wide = (reinterpret_cast<uintptr_t>(y) % 16 == 0 && rows % (mode == HKHIP_SILU_MUL ? 8 : 4) == 0) ? 1 : 0;
-    // The largest tile that still gives most of the 256 CUs a workgroup.
-    auto blocks = [&](uint32_t nw, uint32_t tt) {
-        return ((rows + 32 * nw - 1) / (32 * nw)) * ((n + 32 * tt - 1) / (32 * tt));
-    };
-    // Below that, K slices give the SIMDs a second wave (measured at 512 tokens: 4096x14336
-    // 104 -> 87 us with two slices, 1024x3072 16.8 -> 10.7 us with four).
-    const uint32_t nsb = cols / 256;
-    if (t == HKHIP_Q5_K) // mm2_supports: these two tiles only (two K slices would not fit the LDS)
-        return blocks(8, 4) >= 192 ? launch_mm2_reg<8, 4, HKHIP_Q5_K>(a, s) : launch_mm2_cfg<4, 2, 2, 1, HKHIP_Q5_K>(a, s);
-    if (blocks(8, 4) >= 192) return launch_mm2_reg<8, 4>(a, s);
-    // Two K slices only while the grid stays within one workgroup per CU: a 512-thread workgroup
-    // leaves no room for a second, so past 256 the grid runs in two rounds (6144x1024 at 512
-    // tokens: 19.1 us with two slices, 15.9 with one).
-    if (blocks(4, 2) >= 160)
-        return nsb >= 4 && blocks(4, 2) <= 256 ? launch_mm2_cfg<4, 2, 2, 2>(a, s) : launch_mm2_cfg<4, 2, 2>(a, s);
-    if (blocks(2, 1) >= 128) {
-        if (nsb >= 8) return launch_mm2_cfg<2, 1, 2, 4>(a, s);
-        if (nsb >= 2) return launch_mm2_cfg<2, 1, 2, 2>(a, s);
-        return launch_mm2_cfg<2, 1, 3>(a, s);
-    }
-    return launch_mm2_cfg<1, 1, 3>(a, s);
+    return t == HKHIP_Q5_K ? launch_mm2_reg<8, 4, HKHIP_Q5_K>(a, s) : launch_mm2_reg<8, 4>(a, s);
 }
 
 } // namespace hkhip

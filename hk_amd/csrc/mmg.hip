@@ -1,11 +1,16 @@
-// Prefill GEMM of the super-block formats whose group scales fold into int8 weights: Q6_K, Q3_K
-// and Q2_K (K a multiple of 256).
+// Prefill GEMM of the super-block formats whose group scales fold into int8 weights: Q4_K, Q5_K, Q6_K,
+// Q3_K and Q2_K (K a multiple of 256).
 //
 // Integer arithmetic as in hk's CPU kernels (src/quant/gemm.zig kernelK 180-236 with the canonical
 // unpack of unpack.zig; dotCanonK, vecdot.zig:686-705): per row r, token t and super-block b the
 // products of the 256 weights are one exact integer, scaled once in f32.
 //  * Q6_K: w = sc*(q - 32) in [-4096, 4096] as two int8 planes, 4*w = 256*H + L (q6k_planes); the
 //    two MFMA chains give (H-sum << 8) + L-sum = 4*I, and y += (d/4)*da * that.
+//  * Q4_K: the 6-bit scale sc = 8*sh + sl, planes sh*q and sl*q (each at most 105: one packed 16-bit
+//    multiply makes four weights); I = 8 * (sh-sum) + (sl-sum). Q5_K: sc*q <= 1953 = 256*H + L. The
+//    mins are J = sum_s mn[s]*bsum32[s], an integer below 2^22 whose factors are exact bf16 integers
+//    once bsum32 = 64*u + v (the activation buffer's k_mb plane): one 32x32x16 bf16 MFMA yields J
+//    exactly in f32; y += da*(d*I - dmin*J).
 //  * Q3_K: w = sc*(q - 4), sc in [-32, 31], q in [0, 7]: -w lies in [-128, 124], one int8 plane,
 //    looked up: a group's eight products are two registers, a byte permute picks four at once.
 //    y += -d*da * sum.
@@ -29,7 +34,10 @@
 // Measured at 512 tokens: Q3_K 14336 x 4096 30.6 ms (decode passes of 8 tokens on float-decoded
 // weights) -> 53 us, Q2_K 57 us (1050 TOPS); Q6_K, against a tile that rebuilt its planes every 64
 // tokens with one wave per SIMD, 14336 x 4096 169 -> 82 us, 4096 x 14336 152 -> 105 us, at 100 tokens
-// 90 -> 44 us, 1024 x 4096 29.4 -> 15.9 us. (A three-slot ring with the barrier moved inside the step and
+// 90 -> 44 us, 1024 x 4096 29.4 -> 15.9 us; Q4_K, against a tile with weights loaded row by row into registers
+// and the mins on three bf16 MFMAs, 14336 x 4096 83 -> 73 us, 28672 x 4096 170 -> 158 us (and half the
+// error against float64: 2.0e-7 -> 0.9e-7); Q5_K 14336 x 4096 108 -> 89 us, 4096 x 14336 147 -> 105 us, 4096 x
+// 4096 at 100 tokens 38 -> 15 us. (A three-slot ring with the barrier moved inside the step and
 // the planes built one super-block ahead was no faster, 109 -> 114 us at 4096 x 14336: neither the
 // barrier nor the loads' latency is what bounds it.)
 // MFMA roles: A = activations (tokens as M), B = weights (rows as N); output lane l holds row l%32
@@ -48,6 +56,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef unsigned short us2 __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef short v8s __attribute__((ext_vector_type(8)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 // RB: quant-plane bytes per row and super-block; SB: side bytes.
 template <int T> struct Fmt;
@@ -63,22 +72,44 @@ template <> struct Fmt<HKHIP_Q2_K> {
     static constexpr uint32_t RB = 64, SB = 20;
     static constexpr int planes = 1;
 };
+template <> struct Fmt<HKHIP_Q4_K> {
+    static constexpr uint32_t RB = 144, SB = 0;
+    static constexpr int planes = 2;
+};
+template <> struct Fmt<HKHIP_Q5_K> {
+    static constexpr uint32_t RB = 176, SB = 0;
+    static constexpr int planes = 2;
+};
+// Formats with a min per 32 weights.
+template <int T> constexpr bool has_mins = T == HKHIP_Q4_K || T == HKHIP_Q5_K;
 
 // Activations of one super-block: chunk c of token t at c ^ (t & 15), token scales, and (Q2_K) the
 // tokens' sixteen 16-value sums.
 template <int T, int TOK> struct ASlot {
     int8_t a[TOK * 256];
     float da[(TOK + 63) / 64 * 64];
-    int16_t bs[T == HKHIP_Q2_K ? TOK * 16 : 8];
+    int16_t bs[T == HKHIP_Q2_K || has_mins<T> ? TOK * 16 : 8]; // Q4_K, Q5_K: k_mb's 16 bf16
 };
 // One wave's 32 rows of one super-block.
 template <int T> struct WSlot {
     uint8_t q[32 * Fmt<T>::RB];
-    uint8_t s[T == HKHIP_Q6_K ? 256 : (32 * Fmt<T>::SB + 1023) / 1024 * 1024];
+    uint8_t s[T == HKHIP_Q6_K ? 256 : Fmt<T>::SB ? (32 * Fmt<T>::SB + 1023) / 1024 * 1024 : 16];
 };
+// Two workgroups share a CU's LDS and SIMDs in the tiles of four waves with at most two K slices.
+template <int NW, int KS> constexpr int resident() { return NW * KS < 8 && KS < 4 ? 2 : 1; }
+// Weight buffers per wave: two, so that the next block's loads go out at the start of a step, for the
+// 32-token tiles, whose steps are too short for them otherwise, and for Q4_K (6144 x 14336 at 512 tokens 139
+// -> 131 us; the other formats' larger tiles measured the same or, Q3_K, up to 10 % slower so), where
+// they fit.
+template <int T, int NW, int TT, int KS> constexpr int wbufs() {
+    return (TT == 1 || T == HKHIP_Q4_K) &&
+                   sizeof(ASlot<T, 32 * TT>) * 2 * KS + sizeof(WSlot<T>) * 2 * KS * NW <= 160 * 1024 / resident<NW, KS>()
+               ? 2
+               : 1;
+}
 template <int T, int NW, int TT, int KS> struct Smem {
     ASlot<T, 32 * TT> a[KS][2];
-    WSlot<T> w[KS * NW];
+    WSlot<T> w[KS * NW][wbufs<T, NW, TT, KS>()];
 };
 
 struct MgArgs {
@@ -88,6 +119,7 @@ struct MgArgs {
     const int8_t *aqs;
     const float *ad;
     const int16_t *abs;
+    const uint8_t *amb; // k_mb: per token and super-block 64*u and v of its sub-block sums as bf16
     float *y;
     const float *bias;
     int mode;
@@ -109,16 +141,23 @@ template <> struct Raw<HKHIP_Q6_K> {
 template <> struct Raw<HKHIP_Q3_K> {
     uint4 q[2], hm, side; // side: scales[12], d
 };
+template <> struct Raw<HKHIP_Q4_K> {
+    uint4 hd, q[4];
+};
+template <> struct Raw<HKHIP_Q5_K> {
+    uint4 hd, q[4], x; // x: the fifth bits
+};
 template <> struct Raw<HKHIP_Q2_K> {
     uint4 q[2];
     uint32_t sc[4], dm;
 };
 
 template <int T, int NW, int TT, int KS>
-__global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel(MgArgs a) {
+__global__ __launch_bounds__(NW * KS * 64, (NW * KS * resident<NW, KS>() / 4)) void mmg_kernel(MgArgs a) {
     using F = Fmt<T>;
     constexpr int TOK = 32 * TT;
-    constexpr bool q6 = T == HKHIP_Q6_K, q3 = T == HKHIP_Q3_K, q2 = T == HKHIP_Q2_K;
+    constexpr bool q6 = T == HKHIP_Q6_K, q3 = T == HKHIP_Q3_K, q2 = T == HKHIP_Q2_K, q4 = T == HKHIP_Q4_K,
+                   q5 = T == HKHIP_Q5_K, km = has_mins<T>;
     __shared__ __attribute__((aligned(16))) Smem<T, NW, TT, KS> S;
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wall = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -156,18 +195,19 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
     }
     // Token scales: wave m < TOK/64 loads tokens 64m..; Q2_K's sums: wave m loads tokens 32m...
     const uint32_t doff = clamp_tok(t0 + 64 * wave + lane) * nsb * 4;
-    const uint32_t boff = clamp_tok(t0 + 32 * wave + lane / 2) * (K / 16) * 2 + 16 * (lane & 1);
+    const uint32_t boff = clamp_tok(t0 + 32 * wave + lane / 2) * nsb * 32 + 16 * (lane & 1); // 32 bytes per super-block
     auto issue_a = [&](uint32_t sb, ASlot<T, TOK> &A) {
         const int8_t *ga = a.aqs + 256 * sb;
 #pragma unroll
         for (uint32_t i = 0; i < TPW / 4; i++) load_lds16(ga + aoff[i], &A.a[(TPW * wave + 4 * i) * 256]);
         if (64 * wave < uint32_t(TOK)) load_lds4(reinterpret_cast<const uint8_t *>(a.ad) + doff + 4 * sb, &A.da[64 * wave]);
-        if constexpr (q2) {
+        if constexpr (q2 || km) {
+            const uint8_t *gb = km ? a.amb : reinterpret_cast<const uint8_t *>(a.abs);
 #pragma unroll
             for (uint32_t b = 0; b < (TT + NW - 1) / NW; b++) {
                 const uint32_t m = wave + NW * b;
-                const uint32_t o = b == 0 ? boff : clamp_tok(t0 + 32 * m + lane / 2) * (K / 16) * 2 + 16 * (lane & 1);
-                if (m < uint32_t(TT)) load_lds16(reinterpret_cast<const uint8_t *>(a.abs) + o + 32 * sb, &A.bs[512 * m]);
+                const uint32_t o = b == 0 ? boff : clamp_tok(t0 + 32 * m + lane / 2) * nsb * 32 + 16 * (lane & 1);
+                if (m < uint32_t(TT)) load_lds16(gb + o + 32 * sb, &A.bs[512 * m]);
             }
         }
     };
@@ -198,10 +238,10 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
             soff[i] = clamp_row(rw0 + e / 5) * nsb * 20 + 4 * (e % 5);
         }
     } else {
-        soff[0] = q6 ? srow * nsb : srow * nsb * 16;
+        soff[0] = q6 ? srow * nsb : srow * nsb * 16; // (unused by Q4_K and Q5_K)
     }
-    WSlot<T> &W = S.w[wall];
-    auto issue_w = [&](uint32_t sb) {
+    constexpr int WB = wbufs<T, NW, TT, KS>();
+    auto issue_w = [&](uint32_t sb, WSlot<T> &W) {
         const uint8_t *gw = a.w + uint64_t(sb) * F::RB;
 #pragma unroll
         for (uint32_t i = 0; i < W16; i++) load_lds16(gw + woff[i], &W.q[1024 * i]);
@@ -211,7 +251,7 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
             load_lds4(a.ws + (((soff[0] + sb) >> 1) << 2), &W.s[0]);
         } else if constexpr (q3) {
             load_lds16(a.ws + soff[0] + 16 * sb, &W.s[0]);
-        } else {
+        } else if constexpr (q2) {
 #pragma unroll
             for (uint32_t i = 0; i < 3; i++) load_lds4(a.ws + soff[i] + 20 * sb, &W.s[256 * i]);
         }
@@ -230,7 +270,7 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
         return sb < nsb ? sb : nsb - 1;
     };
     issue_a(sb_of(0), S.a[ks][0]);
-    issue_w(sb_of(0));
+    issue_w(sb_of(0), S.w[wall][0]);
     __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
     __syncthreads();
 
@@ -238,7 +278,12 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
     auto step = [&](uint32_t buf, uint32_t st) {
         ASlot<T, TOK> &A = S.a[ks][buf];
         const uint32_t sb = sb_of(st);
-        issue_a(sb_of(st + 1), S.a[ks][buf ^ 1]);
+        const WSlot<T> &W = S.w[wall][WB == 2 ? buf : 0];
+        const bool more = st + 1 < nst;
+        if (more) {
+            issue_a(sb_of(st + 1), S.a[ks][buf ^ 1]);
+            if constexpr (WB == 2) issue_w(sb_of(st + 1), S.w[wall][buf ^ 1]);
+        }
         // This lane's row half, raw; then the buffer is free for the next super-block.
         Raw<T> R;
         const uint8_t *blk = &W.q[F::RB * j];
@@ -256,6 +301,11 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
             R.q[0] = ld16(blk + 32 + 16 * h);
             R.q[1] = ld16(blk + 64 + 16 * h);
             R.side = ld16(&W.s[16 * j]);
+        } else if constexpr (km) {
+            R.hd = ld16(blk);
+#pragma unroll
+            for (int p = 0; p < 4; p++) R.q[p] = ld16(blk + (q5 ? 48 : 16) + 32 * p + 16 * h);
+            if constexpr (q5) R.x = ld16(blk + 16 + 16 * h);
         } else {
             R.q[0] = ld16(blk + 16 * h);
             R.q[1] = ld16(blk + 32 + 16 * h);
@@ -264,8 +314,10 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
             for (int i = 0; i < 4; i++) R.sc[i] = sd[i];
             R.dm = sd[4];
         }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the reads are done: the bytes may be overwritten
-        issue_w(sb_of(st + 1));
+        if constexpr (WB == 1) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the reads are done: the bytes may be overwritten
+            if (more) issue_w(sb_of(st + 1), S.w[wall][0]);
+        }
         if (KS > 1 && ks + KS * st >= nsb) { // a slice past its last super-block keeps its loads in step
             __builtin_amdgcn_s_waitcnt(0x0F70);
             __syncthreads();
@@ -276,11 +328,28 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
         v4i P[F::planes][8];
         float d;
         v8h mn;           // Q2_K: mins of groups 8h..8h+7
+        v8bf mb;          // Q4_K, Q5_K: the sub-blocks' mins
+        uint32_t scl = 0, sch = 0; // Q4_K, Q5_K: the sub-blocks' scales, a byte each
         float ndmin = 0.0f;
         if constexpr (q6) {
             d = 0.25f * f16_bits_to_f32(((soff[0] + sb) & 1) ? R.d >> 16 : R.d & 0xFFFF);
         } else if constexpr (q3) {
             d = -f16_bits_to_f32(R.side.w & 0xFFFF);
+        } else if constexpr (km) { // the word unpack of vecdot.zig:461-474
+            const uint32_t k1 = 0x3f3f3f3fu, k2 = 0x0f0f0f0fu, k3 = 0x03030303u;
+            scl = R.hd.y & k1;
+            sch = (R.hd.w & k2) | (((R.hd.y >> 6) & k3) << 4);
+            const uint32_t mnl = R.hd.z & k1, mnh = ((R.hd.w >> 4) & k2) | (((R.hd.z >> 6) & k3) << 4);
+            uint32_t w[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const uint32_t src = q < 2 ? mnl : mnh, sh = 16 * (q & 1);
+                const float e = (float)((src >> sh) & 0xFF), o = (float)((src >> (sh + 8)) & 0xFF);
+                w[q] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, o), __builtin_bit_cast(uint32_t, e), 0x07060302u);
+            }
+            mb = __builtin_bit_cast(v8bf, make_uint4(w[0], w[1], w[2], w[3]));
+            d = f16_bits_to_f32(R.hd.x & 0xFFFF);
+            ndmin = -f16_bits_to_f32(R.hd.x >> 16);
         } else {
             const uint32_t m0 = h ? R.sc[2] : R.sc[0], m1 = h ? R.sc[3] : R.sc[1];
 #pragma unroll
@@ -328,6 +397,31 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
                     const uint32_t hb = (c >= 2 ? hw[i] >> (c >= 2 ? c - 2 : 0) : hw[i] << (c < 2 ? 2 - c : 0)) & 0x04040404u;
                     P[0][c][i] = int(__builtin_amdgcn_perm(T1, T0, ((qw[i] >> (2 * p)) & 0x03030303u) | hb));
                 }
+            } else if constexpr (km) {
+                // Sub-block c: nibble c % 2 of qs bytes 32(c/2) + 16h.., fifth bit c of qh bytes 16h...
+                const uint32_t sc = ((c < 4 ? scl : sch) >> (8 * (c % 4))) & 0xFF;
+                const uint4 q4v = R.q[c / 2];
+                const uint32_t qw[4] = {q4v.x, q4v.y, q4v.z, q4v.w};
+                if constexpr (q4) { // sc = 8*sh + sl: planes sh*q and sl*q, each at most 105
+                    const uint32_t fh = (sc >> 3) * 0x00010001u, fl = (sc & 7) * 0x00010001u;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t q = (qw[i] >> (4 * (c % 2))) & 0x0F0F0F0Fu;
+                        P[0][c][i] = int(pk_mul(q, fh));
+                        P[F::planes - 1][c][i] = int(pk_mul(q, fl));
+                    }
+                } else { // sc*q <= 1953 = 256*H + L
+                    const uint4 x = R.x;
+                    const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, m = sc * 0x00010001u;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t b5 = (c > 4 ? xw[i] >> (c > 4 ? c - 4 : 0) : xw[i] << (c < 4 ? 4 - c : 0)) & 0x10101010u;
+                        int hp, lp;
+                        q6k_planes(((qw[i] >> (4 * (c % 2))) & 0x0F0F0F0Fu) | b5, m, 0x00800080u, hp, lp);
+                        P[0][c][i] = hp;
+                        P[F::planes - 1][c][i] = lp;
+                    }
+                }
             } else {
                 // qs bytes 32n + 16h.. bits 2p, scale byte 2c + h (dequant.zig:80-112).
                 const uint32_t sc = (R.sc[c / 2] >> (16 * (c % 2) + 8 * h)) & 0x0F;
@@ -347,7 +441,7 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
 #pragma unroll
         for (int c = 0; c < 4; c++) load_a(0, c);
         v16i comb = {};
-        v16f jt = {};
+        v16f jt = {}; // Q2_K: J; Q4_K, Q5_K: d*I - dmin*J
         // Outputs 2c, 2c + 1 of tile t's update: tokens 32t + 8g + 4h + (0..3), g = c / 2.
         auto update = [&](int t, int c) {
             const float2 dv = *reinterpret_cast<const float2 *>(&A.da[32 * t + 8 * (c / 2) + 4 * h + 2 * (c % 2)]);
@@ -355,7 +449,9 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 const int v = 2 * c + e;
-                if constexpr (q2)
+                if constexpr (km)
+                    acc[t][v] = fmaf(jt[v], ds[e], acc[t][v]);
+                else if constexpr (q2)
                     acc[t][v] = fmaf(fmaf((float)comb[v], d, ndmin * jt[v]), ds[e], acc[t][v]);
                 else
                     acc[t][v] = fmaf((float)comb[v], d * ds[e], acc[t][v]);
@@ -376,9 +472,9 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
                 } else {
                     update(t - 1, c);
                 }
-                if constexpr (q6) s1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[c % 4], P[F::planes - 1][c], s1, 0, 0, 0);
+                if constexpr (F::planes == 2) s1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[c % 4], P[F::planes - 1][c], s1, 0, 0, 0);
                 if (c < 4 || t + 1 < TT) load_a(t, c + 4);
-                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (TT > 1 || !km) __builtin_amdgcn_sched_barrier(0);
             };
             chunk(std::integral_constant<int, 0>{});
             chunk(std::integral_constant<int, 1>{});
@@ -395,8 +491,18 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
                 for (int i = 0; i < 8; i++) bh[i] = (_Float16)b16[i];
                 jt = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh, mn, v16f{}, 0, 0, 0);
             }
+            constexpr int shift = q4 ? 3 : 8;
 #pragma unroll
-            for (int v = 0; v < 16; v++) comb[v] = q6 ? (s0[v] << 8) + s1[v] : s0[v];
+            for (int v = 0; v < 16; v++) s0[v] = F::planes == 2 ? (s0[v] << shift) + s1[v] : s0[v];
+            if constexpr (km) {
+                __builtin_amdgcn_sched_barrier(0); // s1's registers are free for J's tile
+                const uint4 b = ld16(&A.bs[16 * (32 * t + j) + 8 * h]);
+                const v16f jm = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, b), mb, v16f{}, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 16; v++) jt[v] = fmaf((float)s0[v], d, ndmin * jm[v]);
+            } else {
+                comb = s0;
+            }
         }
 #pragma unroll
         for (int c = 0; c < 8; c++) update(TT - 1, c);
@@ -408,9 +514,10 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
         if (st + 1 < nst) step(1, st + 1);
     }
 
-    // The loads of the last step have landed and every wave is past its barrier: the LDS is free.
+    // The loads of the last step have landed and every wave is past its barrier: the LDS is free. (Storing
+    // each tile beside the next one's MFMAs in the last step spilled 200-330 registers in the large tile.)
     float *red = reinterpret_cast<float *>(&S);
-    if constexpr (KS > 1) {
+    if constexpr (KS > 1) { // slices 1.. leave their tiles in the LDS; slice 0 adds them in order
         static_assert((KS - 1) * NW * TT * 4096 <= sizeof(S), "reduction space");
         if (ks > 0) {
 #pragma unroll
@@ -430,17 +537,15 @@ __global__ __launch_bounds__(NW * KS * 64, NW * KS >= 8 ? 2 : 1) void mmg_kernel
         __syncthreads(); // the partial tiles are read: the space takes the output staging
         if (ks > 0) return;
     }
-
     static_assert(NW * 4096 <= sizeof(S), "output staging space");
-    float *st = red + 1024 * wave;
-    const float b = (a.bias && myrow < a.rows) ? a.bias[myrow] : 0.0f;
+    const float bias_r = (a.bias && myrow < a.rows) ? a.bias[myrow] : 0.0f;
 #pragma unroll
     for (int t = 0; t < TT; t++) {
         const uint32_t tk0 = t0 + 32 * t;
         if (a.wide && rw0 + 32 <= a.rows && tk0 + 32 <= a.n)
-            gemm_store_tile_wide(st, acc[t], b, a.y, a.rows, rw0, tk0, a.mode);
+            gemm_store_tile_wide(red + 1024 * wave, acc[t], bias_r, a.y, a.rows, rw0, tk0, a.mode);
         else
-            gemm_store_tile(acc[t], b, a.y, a.rows, a.n, myrow, tk0, a.mode);
+            gemm_store_tile(acc[t], bias_r, a.y, a.rows, a.n, myrow, tk0, a.mode);
     }
 }
 
@@ -453,26 +558,37 @@ template <int T, int NW, int TT, int KS> hipError_t launch_cfg(const MgArgs &a0,
     return hipGetLastError();
 }
 
-// The tile with the fewest rounds of workgroups times what a round costs. Every tile keeps one
-// workgroup on a CU (registers or LDS), so a launch takes ceil(grid / 256) rounds, each a walk over K of
-// the same cost whatever the grid; measured per round at K = 14336, in units of the smallest tile's 29
-// (Q6_K) and 19 us (Q3_K): 7.9 / 7.3, 5.7 / 5.2, 3.1 / 3.0, 1.4 / 1.3 and 1. Over 54 shapes (1024-14336 rows
-// and columns, 16-1000 tokens) the tile chosen so is the fastest of the five or within 10 % of it.
+// The tile whose rounds of workgroups cost least. A round is what is resident at once: one workgroup per
+// CU for the tiles of eight waves (LDS), two for those of four, whose barriers then drift apart. A
+// round costs its super-block steps and its ends (launch or refill, sum over slices, stores), whatever
+// the grid; a two-resident tile's last half round leaves its workgroups a SIMD per wave and costs less.
+// In tenths of a us for Q4_K, measured at 1024-14336 rows, K 1024 and 4096, 36-700 tokens (a round of K 4096:
+// <8,4,1> 60-66 us, <4,2,2> 22-26, <4,2,1> 41 (half 28), <2,1,4> 10-11, <2,1,2> 18 (half 11), <1,1,4> 8.6); the
+// other formats' rounds are in the same ratios within 15 %.
 template <int T> hipError_t launch_fmt(const MgArgs &a, hipStream_t s) {
     constexpr uint32_t CUS = 256;
-    const uint32_t nw[5] = {8, 8, 4, 2, 1}, tt[5] = {4, 2, 2, 1, 1}, cost[5] = {78, 56, 30, 14, 10};
+    struct Tile {
+        uint32_t nw, tt, ks, resident, step, half; // step, half: tenths of a us per super-block step
+    };
+    const Tile tiles[6] = {{8, 4, 1, 1, 37, 37}, {4, 2, 2, 1, 27, 27}, {4, 2, 1, 2, 25, 16},
+                           {2, 1, 4, 1, 22, 22}, {2, 1, 2, 2, 21, 12}, {1, 1, 4, 1, 18, 18}};
+    const uint32_t nsb = a.cols / 256;
     uint64_t best = ~0ull;
     int pick = 0;
-    for (int i = 0; i < 5; i++) {
-        const uint64_t grid = uint64_t((a.rows + 32 * nw[i] - 1) / (32 * nw[i])) * ((a.n + 32 * tt[i] - 1) / (32 * tt[i]));
-        const uint64_t c = (grid + CUS - 1) / CUS * cost[i];
-        if (c < best) best = c, pick = i;
+    for (int i = 0; i < 6; i++) {
+        const Tile &c = tiles[i];
+        const uint64_t grid = uint64_t((a.rows + 32 * c.nw - 1) / (32 * c.nw)) * ((a.n + 32 * c.tt - 1) / (32 * c.tt));
+        const uint64_t cap = CUS * c.resident, rest = grid % cap, steps = (nsb + c.ks - 1) / c.ks;
+        const uint64_t ends = c.ks > 1 ? 15 : 10;
+        const uint64_t cost = grid / cap * (steps * c.step + ends) + (rest == 0 ? 0 : steps * (rest <= CUS ? c.half : c.step) + ends);
+        if (cost < best) best = cost, pick = i;
     }
     switch (pick) {
     case 0: return launch_cfg<T, 8, 4, 1>(a, s);
-    case 1: return launch_cfg<T, 8, 2, 1>(a, s);
-    case 2: return launch_cfg<T, 4, 2, 2>(a, s);
+    case 1: return launch_cfg<T, 4, 2, 2>(a, s);
+    case 2: return launch_cfg<T, 4, 2, 1>(a, s);
     case 3: return launch_cfg<T, 2, 1, 4>(a, s);
+    case 4: return launch_cfg<T, 2, 1, 2>(a, s);
     default: return launch_cfg<T, 1, 1, 4>(a, s);
     }
 }
@@ -480,7 +596,7 @@ template <int T> hipError_t launch_fmt(const MgArgs &a, hipStream_t s) {
 } // namespace mg
 
 bool mmg_supports(int t, uint32_t rows, uint32_t cols, uint32_t n) {
-    if (t != HKHIP_Q6_K && t != HKHIP_Q3_K && t != HKHIP_Q2_K) return false;
+    if (t != HKHIP_Q6_K && t != HKHIP_Q3_K && t != HKHIP_Q2_K && t != HKHIP_Q4_K && t != HKHIP_Q5_K) return false;
     if (cols % 256 != 0 || rows == 0 || n == 0) return false;
     // 32-bit per-lane byte offsets: quant plane, side plane and activations.
     const WLayout W = weight_layout(t, rows, cols);
@@ -501,12 +617,15 @@ hipError_t launch_mmg(int t, const uint8_t *w, uint32_t rows, uint32_t cols, con
     a.aqs = reinterpret_cast<const int8_t *>(xq + A.k_qs);
     a.ad = reinterpret_cast<const float *>(xq + A.k_d);
     a.abs = reinterpret_cast<const int16_t *>(xq + A.k_bs);
+    a.amb = xq + A.k_mb;
     a.y = y;
     a.bias = bias;
     a.mode = mode;
     a.wide = (reinterpret_cast<uintptr_t>(y) % 16 == 0 && rows % (mode == HKHIP_SILU_MUL ? 8 : 4) == 0) ? 1 : 0;
     switch (t) {
     case HKHIP_Q6_K: return mg::launch_fmt<HKHIP_Q6_K>(a, s);
+    case HKHIP_Q4_K: return mg::launch_fmt<HKHIP_Q4_K>(a, s);
+    case HKHIP_Q5_K: return mg::launch_fmt<HKHIP_Q5_K>(a, s);
     case HKHIP_Q3_K: return mg::launch_fmt<HKHIP_Q3_K>(a, s);
     default: return mg::launch_fmt<HKHIP_Q2_K>(a, s);
     }

@@ -1,8 +1,8 @@
-// Prefill GEMM for the 32-weight formats (Q8_0, IQ4_NL, MXFP4, Q4_0, Q4_1, Q5_0, Q5_1), Q5_K and
-// IQ4_XS on the int8 MFMA units (K a multiple of 256).
+// Prefill GEMM for the 32-weight formats (Q8_0, IQ4_NL, MXFP4, Q4_0, Q4_1, Q5_0, Q5_1) and IQ4_XS on
+// the int8 MFMA units (K a multiple of 256).
 //
 // Integer arithmetic as in hk's CPU kernels (src/quant/gemm.zig kernelLegacy 131-176 for the
-// 32-weight blocks, kernelK 180-236 per sub-block for Q5_K and IQ4_XS):
+// 32-weight blocks, kernelK 180-236 per sub-block for IQ4_XS):
 //  * 32-weight formats: y += (dw[r,c]*da[t,c]) * I_c per block c (I_c exact). One 32x32x32
 //    int8 MFMA yields the tile's I_c; then per output one multiply (dw*da), one convert and one
 //    fma. Q4_0 / Q5_0 weights enter as u - zp (kernelLegacy's acci - zp*s); Q4_1 / Q5_1 as u,
@@ -35,27 +35,22 @@ template <int T> struct Fmt;
 template <> struct Fmt<HKHIP_Q8_0> {
     static constexpr uint32_t RB = 256;   // quant-plane bytes per row and step
     static constexpr uint32_t W16 = 8;    // 1-KB direct loads per wave
-    static constexpr uint32_t W4 = 0;     // 256-B direct loads (the rest)
     static constexpr uint32_t WSB = 1024; // scale bytes per wave
     static constexpr uint32_t DAB = 32;   // activation-scale bytes per token and step
 };
 template <> struct Fmt<HKHIP_IQ4_NL> {
-    static constexpr uint32_t RB = 128, W16 = 4, W4 = 0, WSB = 1024, DAB = 32;
+    static constexpr uint32_t RB = 128, W16 = 4, WSB = 1024, DAB = 32;
 };
 template <> struct Fmt<HKHIP_MXFP4> : Fmt<HKHIP_IQ4_NL> {};
 // Q4_0..Q5_1: side data per row and step: d (16 B) and m (16 B) as one 1-KB load per wave (lanes
 // 32-63 take m), the fifth-bit words (32 B) as a second.
 template <int T> struct Fmt4 {
-    static constexpr uint32_t RB = 128, W16 = 4, W4 = 0, WSB = has_qh(T) ? 2048 : 1024, DAB = 32;
+    static constexpr uint32_t RB = 128, W16 = 4, WSB = has_qh(T) ? 2048 : 1024, DAB = 32;
 };
 // IQ4_XS: IQ4_NL's 16 B per 32 weights; the 8-B block header (d, scales_h, scales_l) per row and
 // step as one 4-B load per lane (lane L: row L/2's word L%2).
 template <> struct Fmt<HKHIP_IQ4_XS> {
-    static constexpr uint32_t RB = 128, W16 = 4, W4 = 0, WSB = 256, DAB = 4;
-};
-// Q5_K: hk's 176-B blocks as they are (header, qh[32], qs[128]); rows unswizzled.
-template <> struct Fmt<HKHIP_Q5_K> {
-    static constexpr uint32_t RB = 176, W16 = 5, W4 = 2, WSB = 16, DAB = 4;
+    static constexpr uint32_t RB = 128, W16 = 4, WSB = 256, DAB = 4;
 };
 template <> struct Fmt<HKHIP_Q4_0> : Fmt4<HKHIP_Q4_0> {};
 template <> struct Fmt<HKHIP_Q4_1> : Fmt4<HKHIP_Q4_1> {};
@@ -70,10 +65,9 @@ template <int T, int TOK, int NW, bool MF = true> struct MxSlot {
     uint8_t ws[NW][Fmt<T>::WSB];             // per wave, the rows' f16 scales of the step
     // Activation scales: Q8K per token (wave m fills tokens 64m..64m+63); A8 per block and token,
     // block-major ([8][TOK]), so that four consecutive tokens' scales are one 16-byte read.
-    float da[T == HKHIP_IQ4_XS || T == HKHIP_Q5_K ? 64 * NW : 8 * TOK];
-    // Q5_K: each sub-block's d_a * bsum32; Q4_1 / Q5_1 without MF: the blocks' d_a * s (f32
-    // bits, [8][TOK] as da).
-    uint32_t sa[T == HKHIP_Q5_K || (has_m(T) && !MF) ? 8 * TOK : 1];
+    float da[T == HKHIP_IQ4_XS ? 64 * NW : 8 * TOK];
+    // Q4_1 / Q5_1 without MF: the blocks' d_a * s (f32 bits, [8][TOK] as da).
+    uint32_t sa[has_m(T) && !MF ? 8 * TOK : 1];
     // Q4_1 / Q5_1: the blocks' d_a * s as three bf16 parts, [token][part][8] (a8_dsb), in 1-KB
     // chunks, one load per wave (waves past the last chunk load it again).
     uint32_t dsb[has_m(T) && MF ? 256 * ((TOK * 48 + 1023) / 1024) : 0];
@@ -87,7 +81,6 @@ struct MxArgs {
     const float *ad;
     const float *ads;    // A8 d * s per block (Q4_1, Q5_1)
     const uint8_t *adsb; // the same in bf16 parts, [k/256][n][48 B]
-    const float *adb;   // Q8K d * bsum32 per sub-block (Q5_K)
     float *y;
     const float *bias;
     int mode;
@@ -105,10 +98,7 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
     constexpr bool mf = has_m(T) && KS == 1; // offset term on MFMAs
     using Slot = MxSlot<T, TOK, NW, KS == 1>;
     constexpr bool xs = (T == HKHIP_IQ4_XS);
-    constexpr bool k5 = (T == HKHIP_Q5_K);
-    constexpr bool kqa = xs || k5; // Q8K activations: one scale per token and super-block
-    constexpr bool unswz = k5;           // rows not a power of two of pieces: no swizzle, word tail
-    constexpr uint32_t DBS = 8 * TOK / (64 * NW); // Q5_K: bsum-pair loads per wave
+    constexpr bool kqa = xs; // Q8K activations: one scale per token and super-block
     static_assert(NB == 2 || NB == 3, "ring depth");
     static_assert(kqa ? TOK <= 64 * NW : (8 * TOK) % (64 * NW) == 0, "token scales per wave");
     __shared__ __attribute__((aligned(16))) Slot ring0[KS];
@@ -152,28 +142,18 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
     constexpr uint32_t TPW = TOK / NW; // token rows per wave
     static_assert(TPW % 4 == 0, "token rows per wave");
     constexpr uint32_t DAL = kqa ? 1 : 8 * TOK / (64 * NW);        // token-scale loads per wave
-    constexpr uint32_t CPW = TPW / 4 + F::W16 + F::W4 + (k5 ? 0 : 1) + DAL + (has_qh(T) ? 1 : 0) + (mf ? 1 : has_m(T) ? DAL : 0) +
-                             (k5 ? DBS : 0);
+    constexpr uint32_t CPW = TPW / 4 + F::W16 + 1 + DAL + (has_qh(T) ? 1 : 0) + (mf ? 1 : has_m(T) ? DAL : 0);
     // Weights: 16-byte piece P = 64*i + lane of the wave's area is row P/(RB/16), piece P%(RB/16);
     // rows of 256 or 128 bytes are swizzled (piece c of row r at c ^ (r & 15), resp. r & 7) so
-    // the 32 rows one operand read covers hit distinct banks. Q5_K's 176-byte rows need no
-    // swizzle; its last 512 bytes go as words.
+    // the 32 rows one operand read covers hit distinct banks.
     constexpr uint32_t PPR = F::RB / 16;
-    uint32_t woff[F::W16 + F::W4];
+    uint32_t woff[F::W16];
 #pragma unroll
     for (uint32_t i = 0; i < F::W16; i++) {
         const uint32_t P = 64 * i + lane, lr = P / PPR, pc = P % PPR;
         const uint32_t rr = clamp_row(r0 + 32 * wave + lr);
-        const uint32_t c = unswz ? pc : (pc ^ (lr & (PPR - 1)));
+        const uint32_t c = pc ^ (lr & (PPR - 1));
         woff[i] = rr * nsb * F::RB + 16 * c;
-    }
-    if constexpr (unswz) {
-#pragma unroll
-        for (uint32_t i = 0; i < F::W4; i++) {
-            const uint32_t Wd = 64 * 4 * F::W16 + 64 * i + lane; // 4-byte word of the wave's area
-            const uint32_t rr = clamp_row(r0 + 32 * wave + Wd / (F::RB / 4));
-            woff[F::W16 + i] = rr * nsb * F::RB + 4 * (Wd % (F::RB / 4));
-        }
     }
     // Scales: the blocks' eight f16 (16 bytes) per row and step. Lanes 32-63 repeat lanes 0-31.
     // Q4_0..Q5_1 (side plane per row: d[nbr], m[nbr], qh[nbr]): lanes 32-63 load m, and the
@@ -185,16 +165,6 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
     const uint32_t sbase = !low4 ? srow * G.stride : sidebase + (h && has_m(T) ? G.m_off : 0);
     const uint32_t qhbase = sidebase + G.qh_off + 16 * h;
     const uint32_t xsoff = clamp_row(r0 + 32 * wave + lane / 2) * nsb * 8 + 4 * (lane % 2);
-    // Q5_K d_a * bsum32: load i of wave m covers entries 64*(DBS*m + i) .. of [8][TOK]: sub-block
-    // e / TOK, token e % TOK.
-    uint32_t boff[k5 ? DBS : 1];
-    if constexpr (k5) {
-#pragma unroll
-        for (uint32_t i = 0; i < DBS; i++) {
-            const uint32_t e = 64 * (DBS * wave + i) + lane;
-            boff[i] = clamp_tok(t0 + e % TOK) * (K / 32) * 4 + 4 * (e / TOK);
-        }
-    }
     // Token data: activation int8 rows, swizzled like the weights; token scales.
     uint32_t aoff[TPW / 4];
 #pragma unroll
@@ -233,17 +203,10 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
         const uint8_t *gw = a.w + uint64_t(sb) * F::RB;
 #pragma unroll
         for (uint32_t i = 0; i < F::W16; i++) load_lds16(gw + woff[i], &S.w[wave][1024 * i]);
-#pragma unroll
-        for (uint32_t i = 0; i < F::W4; i++) load_lds4(gw + woff[F::W16 + i], &S.w[wave][1024 * F::W16 + 256 * i]);
         const uint8_t *gd = reinterpret_cast<const uint8_t *>(a.ad);
         if constexpr (xs) {
             load_lds4(a.ws + xsoff + 8 * sb, &S.ws[wave][0]);
             load_lds4(gd + doff[0] + 4 * sb, &S.da[64 * wave]);
-        } else if constexpr (k5) {
-            load_lds4(gd + doff[0] + 4 * sb, &S.da[64 * wave]);
-            const uint8_t *gb = reinterpret_cast<const uint8_t *>(a.adb);
-#pragma unroll
-            for (uint32_t i = 0; i < DBS; i++) load_lds4(gb + boff[i] + 32 * sb, &S.sa[64 * (DBS * wave + i)]);
         } else {
             load_lds16(a.ws + sbase + 16 * sb, &S.ws[wave][0]);
             if constexpr (has_qh(T)) load_lds16(a.ws + qhbase + 32 * sb, &S.ws[wave][1024]);
@@ -301,32 +264,9 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
             const uint8_t *blk = &S.w[wave][F::RB * j];
             v4i wv[8];
             float dw[8], mw[8];
-            if constexpr (k5) {
-                // Sub-block c of this lane's row half: nibble c%2 of qs bytes 32(c/2) + 16h.., fifth
-                // bit c of qh bytes 16h.. (k4Block has_high); scales and mins by the word unpack
-                // (vecdot.zig:461-474).
-                const uint4 hd = *reinterpret_cast<const uint4 *>(blk);
-                const uint4 qh4 = *reinterpret_cast<const uint4 *>(blk + 16 + 16 * h);
-                const uint32_t qhw[4] = {qh4.x, qh4.y, qh4.z, qh4.w};
-                const uint32_t k1 = 0x3f3f3f3fu, k2 = 0x0f0f0f0fu, k3 = 0x03030303u;
-                const uint32_t scw[2] = {hd.y & k1, (hd.w & k2) | (((hd.y >> 6) & k3) << 4)};
-                const uint32_t mnw[2] = {hd.z & k1, ((hd.w >> 4) & k2) | (((hd.z >> 6) & k3) << 4)};
-                const float d = f16_bits_to_f32(hd.x & 0xFFFF), dmin = f16_bits_to_f32(hd.x >> 16);
-#pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    const uint4 x = *reinterpret_cast<const uint4 *>(blk + 48 + 32 * (c / 2) + 16 * h);
-                    const uint32_t xw[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        wv[c][i] = int(((xw[i] >> (4 * (c & 1))) & 0x0F0F0F0Fu) | (((qhw[i] >> c) & 0x01010101u) << 4));
-                    dw[c] = d * (float)((scw[c / 4] >> (8 * (c % 4))) & 0xFF);
-                    mw[c] = dmin * (float)((mnw[c / 4] >> (8 * (c % 4))) & 0xFF);
-                }
-            }
 #pragma unroll
             for (int c = 0; c < 8; c++) {
-                if constexpr (k5) {
-                } else if constexpr (T == HKHIP_Q8_0) {
+                if constexpr (T == HKHIP_Q8_0) {
                     wv[c] = *reinterpret_cast<const v4i *>(blk + 16 * ((2 * c + h) ^ sw));
                 } else {
                     const uint4 x = *reinterpret_cast<const uint4 *>(blk + 16 * (c ^ (j & 7)));
@@ -369,8 +309,7 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
                 mB2 = __builtin_bit_cast(v8bf, make_uint4(ml[0], ml[1], ml[2], ml[3]));
                 mB3 = h ? v8bf{} : mB1;
             }
-            if constexpr (k5) {
-            } else if constexpr (xs) {
+            if constexpr (xs) {
                 // d * ls_c (exact in f32): ls_c = scales_l nibble | scales_h bits << 4, minus 32
                 // (dequant.zig:443-447).
                 const uint2 hd = *reinterpret_cast<const uint2 *>(&S.ws[wave][8 * j]);
@@ -393,7 +332,7 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
                 for (int c = 0; c < 8; c++) {
                     const v16i p = __builtin_amdgcn_mfma_i32_32x32x32_i8(av[c], wv[c], v16i{}, 0, 0, 0);
                     // Scales of this lane's 16 outputs: tokens 32t + 8g + 4h + (0..3).
-                    const float4 *dap = reinterpret_cast<const float4 *>(&S.da[(xs || k5 ? 0 : c * TOK) + 32 * t + 4 * h]);
+                    const float4 *dap = reinterpret_cast<const float4 *>(&S.da[(xs ? 0 : c * TOK) + 32 * t + 4 * h]);
 #pragma unroll
                     for (int g = 0; g < 4; g++) {
                         const float4 dv = dap[2 * g];
@@ -406,12 +345,6 @@ __global__ __launch_bounds__(NW * KS * 64, 1) void mmx_kernel(MxArgs a) {
                             const float dss[4] = {sv.x, sv.y, sv.z, sv.w};
 #pragma unroll
                             for (int e = 0; e < 4; e++) acc[t][4 * g + e] = fmaf(mw[c], dss[e], acc[t][4 * g + e]);
-                        }
-                        if constexpr (k5) { // - dmin * mn_c * (da * bsum32_c)
-                            const float4 bv = *reinterpret_cast<const float4 *>(&S.sa[c * TOK + 32 * t + 4 * h + 8 * g]);
-                            const float db[4] = {bv.x, bv.y, bv.z, bv.w};
-#pragma unroll
-                            for (int e = 0; e < 4; e++) acc[t][4 * g + e] = fmaf(-mw[c], db[e], acc[t][4 * g + e]);
                         }
                     }
                 }
@@ -521,7 +454,7 @@ template <int T> hipError_t launch_low4(const MxArgs &a, hipStream_t s, uint32_t
 } // namespace mx
 
 bool mmx_supports(int t, uint32_t rows, uint32_t cols, uint32_t n) {
-    if (t != HKHIP_IQ4_XS && t != HKHIP_Q5_K && !legacy32(t)) return false;
+    if (t != HKHIP_IQ4_XS && !legacy32(t)) return false;
     if (cols % 256 != 0 || rows == 0 || n == 0) return false;
     // 32-bit per-lane byte offsets: quant plane, scale plane and activations.
     const WLayout W = weight_layout(t, rows, cols);
@@ -533,7 +466,7 @@ hipError_t launch_mmx(int t, const uint8_t *w, uint32_t rows, uint32_t cols, con
     if (!mmx_supports(t, rows, cols, n)) return hipErrorInvalidValue;
     const WLayout W = weight_layout(t, rows, cols);
     const ActLayout A = act_layout(n, cols);
-    const bool kq = act_kind(t) == HKHIP_ACT_Q8K; // Q5_K, IQ4_XS
+    const bool kq = act_kind(t) == HKHIP_ACT_Q8K; // IQ4_XS
     mx::MxArgs a{};
     a.w = w;
     a.ws = w + W.scale_off;
@@ -544,7 +477,6 @@ hipError_t launch_mmx(int t, const uint8_t *w, uint32_t rows, uint32_t cols, con
     a.ad = reinterpret_cast<const float *>(xq + (kq ? A.k_d : A.a8_d));
     a.ads = reinterpret_cast<const float *>(xq + A.a8_ds);
     a.adsb = xq + A.a8_dsb;
-    a.adb = reinterpret_cast<const float *>(xq + A.k_db);
     a.y = y;
     a.bias = bias;
     a.mode = mode;
@@ -563,9 +495,6 @@ hipError_t launch_mmx(int t, const uint8_t *w, uint32_t rows, uint32_t cols, con
     case HKHIP_Q4_1: return mx::launch_low4<HKHIP_Q4_1>(a, s, blocks(8, 2), blocks(4, 2));
     case HKHIP_Q5_0: return mx::launch_low4<HKHIP_Q5_0>(a, s, blocks(8, 2), blocks(4, 2));
     case HKHIP_Q5_1: return mx::launch_low4<HKHIP_Q5_1>(a, s, blocks(8, 2), blocks(4, 2));
-    case HKHIP_Q5_K: // the offset term makes it Q4_1-like; two K slices do not fit with 176-B rows
-        if (blocks(4, 2) >= 160) return mx::launch_cfg<HKHIP_Q5_K, 4, 2, 2>(a, s);
-        return mx::launch_cfg<HKHIP_Q5_K, 4, 1, 2>(a, s);
     case HKHIP_IQ4_XS:
         if (blocks(8, 2) >= 224) return mx::launch_cfg<HKHIP_IQ4_XS, 8, 2, 2>(a, s);
         if (blocks(4, 2) >= 128 && cols >= 1024) return mx::launch_cfg<HKHIP_IQ4_XS, 4, 2, 2, 2>(a, s);

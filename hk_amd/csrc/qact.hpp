@@ -27,13 +27,12 @@ struct Q8KOut {
     float *d;
     int16_t *bs;
     uint16_t *mb;
-    float *db;
     QactIl il;
 };
 // Block b of the input, quantized by one wave (r: this lane's part).
 __device__ __forceinline__ void q8k_out(const Q8KOut &o, uint64_t b, uint32_t lane, const Q8KQ &r) {
     int8_t *qs = o.qs;
-    float *dout = o.d, *dbout = o.db;
+    float *dout = o.d;
     int16_t *bsout = o.bs;
     uint16_t *mbout = o.mb;
     const QactIl &il = o.il;
@@ -49,7 +48,6 @@ __device__ __forceinline__ void q8k_out(const Q8KOut &o, uint64_t b, uint32_t la
     if ((lane & 7) == 0) {
         mbout[b * 16 + lane / 8] = mu;
         mbout[b * 16 + 8 + lane / 8] = mv;
-        dbout[b * 8 + lane / 8] = r.d * (float)b32;
     }
     if (il.tiles) {
         const uint32_t b32i = uint32_t(b); // tokens <= SK_MAX_TOKENS: a small index
@@ -70,7 +68,6 @@ __device__ __forceinline__ void q8k_out(const Q8KOut &o, uint64_t b, uint32_t la
 inline Q8KOut q8k_planes(uint8_t *xq, const ActLayout &L, uint32_t n, uint32_t k) {
     return Q8KOut{reinterpret_cast<int8_t *>(xq + L.k_qs), reinterpret_cast<float *>(xq + L.k_d),
                   reinterpret_cast<int16_t *>(xq + L.k_bs), reinterpret_cast<uint16_t *>(xq + L.k_mb),
-                  reinterpret_cast<float *>(xq + L.k_db),
                   QactIl{xq + L.k_il, reinterpret_cast<uint16_t *>(xq + L.k_ilmb), reinterpret_cast<float *>(xq + L.k_ild),
                          L.tiles, n, k / QK_K}};
 }

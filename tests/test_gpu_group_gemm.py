@@ -50,10 +50,10 @@ def products64(t, raw, m, k, x):
 # (rows, K, tokens): each tile of the dispatch (by the rounds its grid takes), with whole and ragged
 # last rows and tokens, K of one super-block, and K slices that end at different super-blocks.
 SHAPES = [(32, 256, 9), (33, 256, 41), (70, 1280, 33), (96, 2304, 64), (1000, 768, 130), (4100, 1024, 65),
-          (8200, 512, 257), (14340, 256, 511)]
+          (8200, 512, 257), (14340, 256, 511), (8200, 512, 700), (8200, 768, 900)]
 
 
-@pytest.mark.parametrize("t", [F.Q6_K, F.Q3_K, F.Q2_K])
+@pytest.mark.parametrize("t", [F.Q6_K, F.Q5_K, F.Q4_K, F.Q3_K, F.Q2_K])
 @pytest.mark.parametrize("m,k,n", SHAPES)
 @pytest.mark.parametrize("mode", [STORE, ACCUMULATE, SILU_MUL])
 def test_group_gemm(eng, torch_cuda, t, m, k, n, mode):
