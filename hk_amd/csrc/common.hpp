@@ -290,6 +290,14 @@ __device__ __forceinline__ void load_lds4(const void *g, void *lds) {
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" : : "v"(g), "s"(lds_addr(lds)) : "memory", "m0");
 }
 
+// The same from a uniform base and a 32-bit byte offset per lane (no 64-bit address per lane to keep).
+__device__ __forceinline__ void load_lds16(const void *base, uint32_t off, void *lds) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds_addr(lds)) : "memory", "m0");
+}
+__device__ __forceinline__ void load_lds4(const void *base, uint32_t off, void *lds) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base), "s"(lds_addr(lds)) : "memory", "m0");
+}
+
 // Output mode HKHIP_SILU_MUL: output i of gate g (row 2i) and up u (row 2i + 1), as
 // shaders/mmvq.comp:186 computes it.
 __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
@@ -349,9 +357,9 @@ hipError_t launch_mmsk_parts(int t, const MvPartDesc *parts, int nparts, uint32_
 bool mmg_supports(int t, uint32_t rows, uint32_t cols, uint32_t n);
 hipError_t launch_mmg(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n, float *y,
                       const float *bias, int mode, hipStream_t s);
-// Prefill GEMM for the 32-weight formats and IQ4_XS (cols a multiple of 256).
-bool mmx_supports(int t, uint32_t rows, uint32_t cols, uint32_t n);
-hipError_t launch_mmx(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n, float *y,
+// Prefill GEMM for the 32-weight formats and IQ4_XS (cols a multiple of 256; Q8_0, IQ4_NL, Q4_0: of 32).
+bool mmb_supports(int t, uint32_t rows, uint32_t cols, uint32_t n);
+hipError_t launch_mmb(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n, float *y,
                       const float *bias, int mode, hipStream_t s);
 hipError_t launch_mm2(int t, const uint8_t *w, uint32_t rows, uint32_t cols, const uint8_t *xq, uint32_t n, float *y,
                       const float *bias, int mode, hipStream_t s);

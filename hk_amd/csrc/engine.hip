@@ -359,37 +359,14 @@ int hkhip_gemm(hkhip_engine *eng, const hkhip_mat *m, const void *xq_dev, float 
     return HKHIP_OK;
 }
 
-// Fewest tokens for which the GEMM beats 8-token matvec passes (measured on MI355X at the
-// Llama-3-8B FFN shapes: a GEMM pass costs about as much at 16 tokens as at 64, while each
-// matvec pass of 8 tokens streams the weights once more).
-static uint32_t gemm_min_tokens(int t, uint32_t rows) {
-    switch (t) {
-    case HKHIP_Q6_K:
-    case HKHIP_Q8_0: return 33;
-    case HKHIP_IQ4_NL: case HKHIP_MXFP4: return 25;
-    case HKHIP_Q5_K: case HKHIP_Q4_0: case HKHIP_Q4_1: case HKHIP_Q5_0: case HKHIP_Q5_1: case HKHIP_IQ4_XS:
-        // Measured at 9-64 tokens: with 14336 rows the GEMM beats two decode passes from 9
-        // tokens; with 4096 rows (K 14336) it costs 50-120 us at any count (Q4_1 50, IQ4_XS 66,
-        // Q5_1 82, Q5_0 98, Q4_0 104, Q5_K 118), which the passes (20-25 us per 8 tokens) reach at
-        // the counts below.
-        if (rows >= 8192) return 9;
-        return t == HKHIP_Q4_1 ? 17 : (t == HKHIP_IQ4_XS || t == HKHIP_Q5_1) ? 25 : t == HKHIP_Q5_0 ? 33 : 41;
-    default: return 9;
-    }
-}
-
 int hkhip_mm(hkhip_engine *eng, const hkhip_mat *m, const void *xq_dev, float *y_dev, uint32_t n,
              const float *bias_dev, int mode) {
-    // The CPU engine tiles from min_tiled_tokens = 8 (matmul.zig:18); here the register matvec
-    // covers up to 8 tokens and, below the GEMM's break-even, runs in passes of 8.
+    // The CPU engine tiles from min_tiled_tokens = 8 (matmul.zig:18). Here the decode kernels take up to 8
+    // tokens; from 9 the GEMM (or the small-batch kernel it leaves Q4_K and Q6_K to up to 32) beats two
+    // passes of them: 14336 x 4096 at 9-16 tokens Q8_0 16 against 42 us, Q5_K 18 against 50, 4096 x 4096 11.6
+    // against 18, 10 against 20.
     if (n <= 8) return hkhip_matvec(eng, m, xq_dev, y_dev, n, bias_dev, mode);
-    if (n >= gemm_min_tokens(m->t, m->rows)) return hkhip_gemm(eng, m, xq_dev, y_dev, n, bias_dev, mode);
-    int rc = enter(eng);
-    if (rc || (rc = check_product(m, xq_dev, y_dev, n, mode)) || (rc = check_prepared(m))) return rc;
-    if (mode == HKHIP_SILU_MUL && bias_dev) return fail(HKHIP_E_BAD_ARGUMENT, "silu(gate)*up takes no bias");
-    HIP_TRY(launch_mmvq(m->t, reinterpret_cast<const uint8_t *>(m->mem), m->rows, m->cols,
-                        reinterpret_cast<const uint8_t *>(xq_dev), n, y_dev, bias_dev, mode, eng->cur), "mmvq launch");
-    return HKHIP_OK;
+    return hkhip_gemm(eng, m, xq_dev, y_dev, n, bias_dev, mode);
 }
 
 int hkhip_mm_noalloc(hkhip_engine *eng, const hkhip_mat *m, const float *x_dev, float *y_dev, uint32_t n,

@@ -298,15 +298,15 @@ hipError_t launch_mm(int t, const uint8_t *w, uint32_t rows, uint32_t cols, cons
     // Few tokens: the weights dominate, so the kernel that streams them (small-batch MFMA); many:
     // the tiled GEMM.
     if (n >= SK_MIN_TOKENS && mmsk_supports(t, rows, cols, n)) return launch_mmsk(t, w, rows, cols, xq, n, y, bias, mode, s);
-    // Below these counts passes of the decode kernel are faster (14336 x 4096 at one token: Q3_K 10.2
-    // against the GEMM's 11.8 us, at four 17.0 against 11.8; MXFP4 9.2 against 38, at 24 about 60 both).
-    if ((n < SK_MIN_TOKENS && (t == HKHIP_Q3_K || t == HKHIP_Q2_K)) || (n <= 24 && t == HKHIP_MXFP4))
+    // Below these counts the decode kernel is faster (14336 x 4096 at one token: Q3_K 10.2 against the
+    // GEMM's 11.8 us, at four 17.0 against 11.8; MXFP4 4096 x 14336 at eight 23 against 33).
+    if ((n < SK_MIN_TOKENS && (t == HKHIP_Q3_K || t == HKHIP_Q2_K)) || (n <= 8 && t == HKHIP_MXFP4))
         return launch_mmvq(t, w, rows, cols, xq, n, y, bias, mode, s);
     if (mm2_supports(t, rows, cols, n)) return launch_mm2(t, w, rows, cols, xq, n, y, bias, mode, s);
     if (mmg_supports(t, rows, cols, n)) return launch_mmg(t, w, rows, cols, xq, n, y, bias, mode, s);
-    if (mmx_supports(t, rows, cols, n)) return launch_mmx(t, w, rows, cols, xq, n, y, bias, mode, s);
-    // Q4_0..Q5_1 rows that are not whole super-blocks, and matrices past the GEMMs' 32-bit offsets: decode
-    // passes of 8 tokens.
+    if (mmb_supports(t, rows, cols, n)) return launch_mmb(t, w, rows, cols, xq, n, y, bias, mode, s);
+    // Q4_1, Q5_0 and Q5_1 rows that are not whole super-blocks, and matrices past the GEMMs' 32-bit offsets:
+    // decode passes of 8 tokens.
     if ((legacy32(t) && t != HKHIP_Q8_0 && t != HKHIP_IQ4_NL) || t == HKHIP_Q3_K || t == HKHIP_Q2_K)
         return launch_mmvq(t, w, rows, cols, xq, n, y, bias, mode, s);
     WLayout W = weight_layout(t, rows, cols);
