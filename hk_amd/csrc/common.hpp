@@ -291,6 +291,8 @@ __device__ __forceinline__ void load_lds4(const void *g, void *lds) {
 }
 
 // The same from a uniform base and a 32-bit byte offset per lane (no 64-bit address per lane to keep).
+// In the GEMM tiles that fill the register file the 64-bit addresses were spilled, and a reload waits for the
+// loads in flight: Q4_K 28672 x 4096 at 512 tokens 161 -> 151 us, Q5_K 175 -> 168 us with this form.
 __device__ __forceinline__ void load_lds16(const void *base, uint32_t off, void *lds) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds_addr(lds)) : "memory", "m0");
 }

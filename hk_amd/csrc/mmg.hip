@@ -199,15 +199,15 @@ __global__ __launch_bounds__(NW * KS * 64, (NW * KS * resident<NW, KS>() / 4)) v
     auto issue_a = [&](uint32_t sb, ASlot<T, TOK> &A) {
         const int8_t *ga = a.aqs + 256 * sb;
 #pragma unroll
-        for (uint32_t i = 0; i < TPW / 4; i++) load_lds16(ga + aoff[i], &A.a[(TPW * wave + 4 * i) * 256]);
-        if (64 * wave < uint32_t(TOK)) load_lds4(reinterpret_cast<const uint8_t *>(a.ad) + doff + 4 * sb, &A.da[64 * wave]);
+        for (uint32_t i = 0; i < TPW / 4; i++) load_lds16(ga, aoff[i], &A.a[(TPW * wave + 4 * i) * 256]);
+        if (64 * wave < uint32_t(TOK)) load_lds4(reinterpret_cast<const uint8_t *>(a.ad) + 4 * sb, doff, &A.da[64 * wave]);
         if constexpr (q2 || km) {
             const uint8_t *gb = km ? a.amb : reinterpret_cast<const uint8_t *>(a.abs);
 #pragma unroll
             for (uint32_t b = 0; b < (TT + NW - 1) / NW; b++) {
                 const uint32_t m = wave + NW * b;
                 const uint32_t o = b == 0 ? boff : clamp_tok(t0 + 32 * m + lane / 2) * nsb * 32 + 16 * (lane & 1);
-                if (m < uint32_t(TT)) load_lds16(gb + o + 32 * sb, &A.bs[512 * m]);
+                if (m < uint32_t(TT)) load_lds16(gb + 32 * sb, o, &A.bs[512 * m]);
             }
         }
     };
@@ -244,16 +244,16 @@ __global__ __launch_bounds__(NW * KS * 64, (NW * KS * resident<NW, KS>() / 4)) v
     auto issue_w = [&](uint32_t sb, WSlot<T> &W) {
         const uint8_t *gw = a.w + uint64_t(sb) * F::RB;
 #pragma unroll
-        for (uint32_t i = 0; i < W16; i++) load_lds16(gw + woff[i], &W.q[1024 * i]);
+        for (uint32_t i = 0; i < W16; i++) load_lds16(gw, woff[i], &W.q[1024 * i]);
 #pragma unroll
-        for (uint32_t i = 0; i < W4; i++) load_lds4(gw + woff[W16 + i], &W.q[1024 * W16 + 256 * i]);
+        for (uint32_t i = 0; i < W4; i++) load_lds4(gw, woff[W16 + i], &W.q[1024 * W16 + 256 * i]);
         if constexpr (q6) {
-            load_lds4(a.ws + (((soff[0] + sb) >> 1) << 2), &W.s[0]);
+            load_lds4(a.ws, ((soff[0] + sb) >> 1) << 2, &W.s[0]);
         } else if constexpr (q3) {
-            load_lds16(a.ws + soff[0] + 16 * sb, &W.s[0]);
+            load_lds16(a.ws + 16 * sb, soff[0], &W.s[0]);
         } else if constexpr (q2) {
 #pragma unroll
-            for (uint32_t i = 0; i < 3; i++) load_lds4(a.ws + soff[i] + 20 * sb, &W.s[256 * i]);
+            for (uint32_t i = 0; i < 3; i++) load_lds4(a.ws + 20 * sb, soff[i], &W.s[256 * i]);
         }
     };
 
