@@ -152,9 +152,8 @@ int hkhip_act_export(hkhip_engine *eng, const void *xq_dev, uint32_t n, uint32_t
  * with hkhip_qact for the matrix's kind (A8: Q8_0, IQ4_NL; Q8K: Q4_K, Q6_K). bias may be NULL.
  * hkhip_matvec: decode kernels, 1 <= n <= 8 (src/kernels_impl.zig:14-33 rows).
  * hkhip_gemm:   prefill MFMA kernels, any n >= 1 (src/quant/gemm.zig tiles).
- * hkhip_mm:     picks matvec for n <= 8, then 8-token matvec passes up to the GEMM's break-even
- *               (Q6_K / Q8_0: 32 tokens, IQ4_NL: 24; Q4_K has none), then gemm (the CPU engine's
- *               switch is matmul.zig:18 min_tiled_tokens = 8).
+ * hkhip_mm:     picks matvec for n <= 8, gemm from 9 tokens (the CPU engine's switch is matmul.zig:18
+ *               min_tiled_tokens = 8).
  * mode is HKHIP_STORE, HKHIP_ACCUMULATE or HKHIP_SILU_MUL. */
 int hkhip_matvec(hkhip_engine *eng, const hkhip_mat *m, const void *xq_dev, float *y_dev, uint32_t n,
                  const float *bias_dev, int mode);
